@@ -155,8 +155,9 @@ int64_t moba_hip_prefill_bwd_work(int n_kv_tiles, int kv_splits, int D);
  * natural log, mapping [M] int64 (row p = t*H + h of each remote partial).
  * out [T,H,D] (dtype) and lse [T,H] fp32: m = max of the row's LSEs,
  * O = (w_self o_self + sum w_j o_j) / z, z = sum w_j + w_self, L = m + log z.
- * Always deterministic and atomic-free: remote partials are taken in
- * ascending j (a stable radix sort by row), merged one wave64 per row.
+ * Always deterministic: a row's remote partials are taken in ascending j
+ * (ordered by integer minima, whose result does not depend on timing; no
+ * floating-point value passes through an atomic).
  * D a multiple of 8 in [8,256], kmax in [1,8].  work: moba_hip_merge_work(T*H,
  * M) bytes.  status [2] int32 (device), written on the stream: status[0] = 1
  * if a mapping entry lies outside [0,T*H) (ignored), status[1] = 1 if a row
@@ -166,6 +167,12 @@ int moba_hip_merge(const void* self_out, const float* self_lse, const void* remo
                    const float* remote_lse, const int64_t* mapping, int dtype, int64_t T, int H,
                    int D, int64_t M, int kmax, void* work, int* status, void* out, float* lse,
                    void* stream);
+
+/* moba_hip_merge with an int32 mapping, read as it is. */
+int moba_hip_merge_i32(const void* self_out, const float* self_lse, const void* remote_out,
+                       const float* remote_lse, const int32_t* mapping, int dtype, int64_t T,
+                       int H, int D, int64_t M, int kmax, void* work, int* status, void* out,
+                       float* lse, void* stream);
 
 /* Bytes of the work buffer of moba_hip_merge for P = T*H rows and M remote
  * partials (-1 for bad sizes).  Shape query; no reference counterpart. */

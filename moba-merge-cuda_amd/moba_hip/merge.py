@@ -2,8 +2,8 @@
 
 Drop-in for ``merge_forward_cuda`` (src/moba_opt/ops/merge_cuda.py:32-60,
 binding src/moba_opt/ops/bindings.cpp:6-22): same arguments, same checks and
-messages, returns ``(O, LSE)``.  The merge itself is ``moba_hip_merge``: no
-atomics, remote partials of a row taken in ascending index order, so the
+messages, returns ``(O, LSE)``.  The merge itself is ``moba_hip_merge``:
+remote partials of a row are taken in ascending index order, so the
 result is always deterministic (``deterministic`` is accepted and documents
 that).  ``check_capacity`` reads two status words after the launch (one small
 device-to-host copy, like the reference's overflow check) and raises.
@@ -69,7 +69,8 @@ def merge_forward(self_out, self_lse, remote_out, remote_lse, mapping, kmax=None
     sl = self_lse.to(torch.float32).contiguous()
     ro = remote_out.reshape(M, D).contiguous()
     rl = remote_lse.to(torch.float32).contiguous()
-    mp = mapping.to(torch.int64).contiguous()
+    mp = mapping.contiguous()
+    entry = "moba_hip_merge_i32" if mp.dtype == torch.int32 else "moba_hip_merge"
     lib = _lib.load()
     nbytes = lib.moba_hip_merge_work(P, M)
     if nbytes < 0:
@@ -79,7 +80,7 @@ def merge_forward(self_out, self_lse, remote_out, remote_lse, mapping, kmax=None
         status = torch.empty(2, dtype=torch.int32, device=dev)
         out = torch.empty_like(so)
         lse = torch.empty((T, H), dtype=torch.float32, device=dev)
-        _lib.call("moba_hip_merge", so.data_ptr(), sl.data_ptr(), ro.data_ptr(), rl.data_ptr(),
+        _lib.call(entry, so.data_ptr(), sl.data_ptr(), ro.data_ptr(), rl.data_ptr(),
                   mp.data_ptr(), _DTYPES[so.dtype], T, H, D, M, kmax, work.data_ptr(),
                   status.data_ptr(), out.data_ptr(), lse.data_ptr(), _lib.stream_of(dev))
         if check_capacity and M:

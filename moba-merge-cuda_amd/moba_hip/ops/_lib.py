@@ -34,6 +34,7 @@ SIGNATURES = {
                              _P, _I, _P, _I, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _P,
                              _P, _P],
     "moba_hip_merge": [_P, _P, _P, _P, _P, _I, _L, _I, _I, _L, _I, _P, _P, _P, _P, _P],
+    "moba_hip_merge_i32": [_P, _P, _P, _P, _P, _I, _L, _I, _I, _L, _I, _P, _P, _P, _P, _P],
     "moba_hip_merge_work": [_L, _L],
     "moba_hip_decode_work_items": [_I, _I, _I],
     "moba_hip_paged_append": [_P, _P, _I, _I, _I, _I, _P, _P, _I, _P, _I, _P, _P, _P],

@@ -105,3 +105,41 @@ def test_merge_capacity_and_range_errors(cuda_device):
             merge_forward(so, sl, ro, rl, torch.tensor(bad, device="cuda"))
     with pytest.raises(ValueError, match="deterministic"):
         merge_forward(so, sl, ro, rl, crowded, deterministic=1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kmax,counts", [(1, (2, 0, 1)), (3, (5, 3, 0, 4)), (4, (9, 4)),
+                                         (8, (300, 8, 1))])
+def test_merge_keeps_the_first_kmax_partials(cuda_device, kmax, counts, dtype):
+    """Rows with fewer, exactly and more remote partials than kmax (up to a
+    row that a whole workgroup of partials meets in): each keeps its kmax
+    lowest indices, in every run, for int32 and int64 mappings, and for inputs
+    whose rows do not start on 16 bytes."""
+    from moba_hip.merge import merge_forward
+    g = torch.Generator().manual_seed(kmax)
+    n, D = len(counts), 40
+    mapping = np.repeat(np.arange(n), counts)
+    np.random.default_rng(kmax).shuffle(mapping)
+    M = len(mapping)
+    step = 4 if dtype == torch.float32 else 2
+
+    def shifted(*shape):   # contiguous, `step * 2` bytes past an aligned start
+        flat = torch.randn(int(np.prod(shape)) + 16, generator=g).to("cuda", dtype)
+        return flat[8 // step:8 // step + int(np.prod(shape))].view(*shape)
+    so, ro = shifted(n, 1, D), shifted(M, D)
+    sl, rl = torch.randn(n, 1, generator=g).cuda(), torch.randn(M, generator=g).cuda()
+    keep = np.concatenate([np.flatnonzero(mapping == r)[:kmax] for r in range(n)]).astype(int)
+    ref = _ref(so, sl, ro[keep], rl[keep], torch.from_numpy(mapping[keep]))
+    first = None
+    for mp in (torch.from_numpy(mapping).cuda(), torch.from_numpy(mapping).int().cuda()):
+        for _ in range(3):
+            out, lse = merge_forward(so, sl, ro, rl, mp, kmax=kmax, check_capacity=False)
+            first = first or (out, lse)
+            assert torch.equal(out, first[0]) and torch.equal(lse, first[1])
+    if dtype == torch.float32:
+        np.testing.assert_allclose(out.double().cpu().numpy(), ref[0], atol=2e-6, rtol=1e-5)
+    else:
+        assert_close_stats(out, ref[0], dtype, "merged out")
+    np.testing.assert_allclose(lse.double().cpu().numpy(), ref[1], atol=2e-6, rtol=1e-6)
+    with pytest.raises(RuntimeError, match="capacity exceeded"):
+        merge_forward(so, sl, ro, rl, mp, kmax=kmax)
