@@ -68,8 +68,8 @@ int moba_hip_route_prefill(const void* q, int dtype, int T, int Hq, int Hkv, int
  * counts] = ((s*Hq + h) << 3) | j where j is the chunk's rank in sel[s,h,:]
  * (R <= 8, T*Hq < 2^28); the partial slot of that row is (s*Hq + h)*R + j.
  * work is an 8-byte aligned int32 workspace of moba_hip_pack_experts_work(T,
- * Hq, Hkv, F) entries (64-bit selection masks of every (token, head), then
- * per-block candidate counts of each expert).
+ * Hq, Hkv, F) entries (counts of every candidate per block of 256 tokens of a
+ * head).
  * Replaces the nonzero/index_select packing of grouped_attention.py:78-94. */
 int moba_hip_pack_experts(const int* sel, int T, int Hq, int Hkv, int R,
                           const int* cu_chunk, const int* chunk_batch, const int* cu_seqlens,
@@ -79,6 +79,17 @@ int moba_hip_pack_experts(const int* sel, int T, int Hq, int Hkv, int R,
 /* Size in int32 entries of the work buffer of moba_hip_pack_experts (-1 for a
  * bad shape).  Helper of the entry above; no counterpart in the reference. */
 int64_t moba_hip_pack_experts_work(int T, int Hq, int Hkv, int F);
+
+/* moba_hip_chunk_means, moba_hip_route_prefill and moba_hip_pack_experts in
+ * one call (the same arguments and results): the gate kernel counts the picks
+ * of its blocks while it has them, so the packing reads them once. */
+int moba_hip_prefill_route(const void* q, const void* k, int dtype, int T, int Hq, int Hkv, int D,
+                           const int* chunk_start, int chunk, int precision,
+                           const int* cu_chunk, int nchunk, const int* chunk_batch,
+                           const int* first_chunk, const int* cu_seqlens, const int* filtered,
+                           int R, int F, int block_rows, float* means, int* sel, float* gate,
+                           int* counts, int* row_off, int* tile_off, int* rows, int* work,
+                           void* stream);
 
 /* Query rows per prefill tile for head dim D (-1 for an unsupported D): the
  * block_rows of moba_hip_pack_experts and the row step of the self tiles

@@ -19,6 +19,30 @@ namespace {
 
 constexpr int kMaxRemote = 8;
 
+// Pick bits of a block of 256 consecutive tokens of one head (thread = token),
+// for the candidates [t0, t0 + kPickRows): word 4 r + w holds the tokens of
+// wave w that picked candidate t0 + r.  A token's rank among the block's picks
+// of a candidate is then a population count, and so is the block's number of
+// picks.  The words are built by OR, which no order changes.  fs: the
+// thread's picks (filtered indices, -1 for none).
+constexpr int kPickRows = 256;
+
+MOBA_DEV void pick_bits(uint64_t* bits, const int (&fs)[kMaxRemote], int t0) {
+  const int tid = threadIdx.x;
+  __syncthreads();  // the words of the tile before are consumed
+#pragma unroll
+  for (int w = 0; w < 4; ++w) bits[4 * tid + w] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kMaxRemote; ++j) {
+    const int r = fs[j] - t0;
+    if (fs[j] >= 0 && r >= 0 && r < kPickRows)
+      atomicOr(reinterpret_cast<unsigned long long*>(bits + 4 * r + (tid >> 6)),
+               1ull << (tid & 63));
+  }
+  __syncthreads();
+}
+
 // One workgroup per (filtered chunk, kv head, dim slice of D / ds).  The mean of dim d is the
 // canonical sum: 64 partial sums s_j over the tokens j, j+64, j+128, ... in
 // increasing order, then the fixed tree canon_tree over j.  Work item
@@ -110,7 +134,8 @@ __global__ __launch_bounds__(256) void route_kernel(const uint16_t* __restrict__
                                                     const int* __restrict__ chunk_batch,
                                                     const int* __restrict__ first_chunk, int R,
                                                     int F, int* __restrict__ sel,
-                                                    float* __restrict__ gate) {
+                                                    float* __restrict__ gate,
+                                                    int* __restrict__ blk_count) {
   __shared__ __attribute__((aligned(16))) float mt[kRouteTile * DP];
   __shared__ int red[2][4];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -229,7 +254,6 @@ __global__ __launch_bounds__(256) void route_kernel(const uint16_t* __restrict__
       if (cnt < R) cnt++;
     }
   }
-  if (!live) return;
   // ascending chunk order for the slot list (static sorting network)
 #pragma unroll
   for (int pass = 0; pass < kMaxRemote; ++pass) {
@@ -238,8 +262,29 @@ __global__ __launch_bounds__(256) void route_kernel(const uint16_t* __restrict__
       if (j + 1 < cnt && ix[j] > ix[j + 1]) { int t = ix[j]; ix[j] = ix[j + 1]; ix[j + 1] = t; }
     }
   }
-  int* out = sel + idx * R;
-  for (int j = 0; j < R; ++j) out[j] = j < cnt ? ix[j] : -1;
+  if (live) {
+    int* out = sel + idx * R;
+    for (int j = 0; j < R; ++j) out[j] = j < cnt ? ix[j] : -1;
+  }
+  if (blk_count == nullptr) return;
+  // this workgroup's count of every candidate, for the expert packing
+  int fs[kMaxRemote];
+#pragma unroll
+  for (int j = 0; j < kMaxRemote; ++j) fs[j] = live && j < cnt ? ix[j] - b : -1;
+  static_assert(kRouteTile * DP * 4 >= kPickRows * 4 * 8, "the means tile holds the pick bits");
+  uint64_t* bits = reinterpret_cast<uint64_t*>(mt);
+  int* dst = blk_count + (int64_t)h * gridDim.x + blockIdx.x;
+  const int64_t fstep = (int64_t)Hq * gridDim.x;
+  for (int f = tid; f < F; f += 256)
+    if (f < flo || f >= fhi) dst[f * fstep] = 0;
+  for (int t0 = flo; t0 < fhi; t0 += kPickRows) {
+    pick_bits(bits, fs, t0);
+    const int f = t0 + tid;
+    if (f < fhi) {
+      const uint64_t* w = bits + 4 * tid;
+      dst[f * fstep] = __popcll(w[0]) + __popcll(w[1]) + __popcll(w[2]) + __popcll(w[3]);
+    }
+  }
 }
 
 __global__ void fill_f32_kernel(float* p, int64_t n, float v) {
@@ -248,168 +293,207 @@ __global__ void fill_f32_kernel(float* p, int64_t n, float v) {
 }
 
 // ---- expert packing ------------------------------------------------------
-// Expert e = f*Hkv + kvh (reference order: (chunk, kv head)).  Its candidate
-// rows are (g, s) for g in the kv group and s from the chunk end to the
-// sequence end, enumerated g-major like the reference's nonzero over
-// [F*Hkv, G*T] (grouped_attention.py:78-80).
+// Expert e = f*Hkv + kvh (reference order: (chunk, kv head)).  Its rows are
+// the (g, s) that picked chunk f, g-major and s ascending, as the reference's
+// nonzero over [F*Hkv, G*T] enumerates them (grouped_attention.py:78-80).
+// Blocks of 256 consecutive tokens of one head are counted per candidate
+// (blk_count[f][h][block]: an expert's blocks are contiguous and in the order
+// of its rows), the counts become offsets within the expert, and each block
+// places its picks: no pass reads more than the picks and the counts.
+// Scanning every candidate row of every expert for its selection bit, in a
+// count and in a fill pass, took 59 us at T 32768, 8 heads, 63 candidates (20
+// here), and 25 us at T 8192, 12 heads, 15 candidates (13 here).  What is left
+// is latency: selection, chunk, offset and row are four dependent accesses
+// (all eight pick slots loaded without branches measured slower, 20 -> 23 us:
+// three of them hold picks).
 
-// Selection bitmasks: word w of row (s, h) has bit f % 64 set when (s, h)
-// selected the chunk of filtered index f, f / 64 == w; laid out
-// mask[(h * NW + w) * T + s], so the candidate scans of the experts, which
-// walk s for a fixed (h, w), read 8 consecutive bytes per candidate instead
-// of a strided R-int row of sel.  One thread per (s, h).
-__global__ __launch_bounds__(256) void sel_mask_kernel(const int* __restrict__ sel, int T, int Hq,
-                                                       int R, const int* __restrict__ chunk_batch,
-                                                       int NW, uint64_t* __restrict__ mask) {
-  const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;  // s * Hq + h
-  if (row >= (int64_t)T * Hq) return;
-  const int s = (int)(row / Hq), h = (int)(row % Hq);
-  int fs[kMaxRemote];
+struct PackArgs {
+  const int* sel;
+  int T, Hq, Hkv, R;
+  const int *cu_chunk, *chunk_batch, *cu_seqlens, *filtered;
+  int F, block_rows;
+  int *counts, *row_off, *tile_off, *rows, *blk;
+};
+
+// Filtered index of each pick of (s, h); -1 for none and for an entry that is
+// not a candidate of the token (a later chunk, another sequence's).  With
+// `at`, also the block's entry of the block counts for each pick; it is
+// loaded beside what the check reads, not after it.
+MOBA_DEV void load_picks(const PackArgs& a, int s, int h, int (&fs)[kMaxRemote],
+                         int (*at)[kMaxRemote] = nullptr, int64_t blk = 0, int nblk = 0) {
+  int c[kMaxRemote], b[kMaxRemote];
+#pragma unroll
+  for (int j = 0; j < kMaxRemote; ++j)
+    c[j] = s < a.T && j < a.R ? a.sel[((int64_t)s * a.Hq + h) * a.R + j] : -1;
+#pragma unroll
+  for (int j = 0; j < kMaxRemote; ++j) b[j] = c[j] >= 0 ? a.chunk_batch[c[j]] : 0;
 #pragma unroll
   for (int j = 0; j < kMaxRemote; ++j) {
-    const int c = j < R ? sel[row * R + j] : -1;
-    fs[j] = c >= 0 ? c - chunk_batch[c] : -1;
+    fs[j] = -1;
+    const int f = c[j] - b[j];
+    if (c[j] < 0 || f >= a.F) continue;
+    const int n = at ? a.blk[((int64_t)f * a.Hq + h) * nblk + blk] : 0;
+    const bool ok = a.filtered[f] == c[j] && s >= a.cu_chunk[c[j] + 1] &&
+                    s < a.cu_seqlens[b[j] + 1];
+    if (ok) fs[j] = f;
+    if (at) (*at)[j] = n;
   }
-  for (int w = 0; w < NW; ++w) {
-    uint64_t m = 0;
+}
+
+// Block counts of an existing selection (the route kernel writes its own).
+__global__ __launch_bounds__(256) void pick_count_kernel(PackArgs a) {
+  __shared__ uint64_t bits[kPickRows * 4];
+  const int tid = threadIdx.x, h = blockIdx.y;
+  int fs[kMaxRemote];
+  load_picks(a, blockIdx.x * 256 + tid, h, fs);
+  for (int t0 = 0; t0 < a.F; t0 += kPickRows) {
+    pick_bits(bits, fs, t0);
+    const int f = t0 + tid;
+    if (f < a.F) {
+      const uint64_t* w = bits + 4 * tid;
+      a.blk[((int64_t)f * a.Hq + h) * gridDim.x + blockIdx.x] =
+          __popcll(w[0]) + __popcll(w[1]) + __popcll(w[2]) + __popcll(w[3]);
+    }
+  }
+}
+
+// Exclusive scan over the 256 threads of a workgroup; total: the sum.
+template <typename I> MOBA_DEV I block_scan_256(I v, I& total, I* part) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  I inc = v;
 #pragma unroll
-    for (int j = 0; j < kMaxRemote; ++j)
-      if (fs[j] >= 0 && (fs[j] >> 6) == w) m |= 1ull << (fs[j] & 63);
-    mask[((int64_t)h * NW + w) * T + s] = m;
+  for (int o = 1; o < 64; o <<= 1) {
+    const I y = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += y;
   }
+  __syncthreads();  // part's earlier use is over
+  if (lane == 63) part[w] = inc;
+  __syncthreads();
+  I before = 0;
+  total = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (i < w) before += part[i];
+    total += part[i];
+  }
+  return before + inc - v;
 }
 
-struct ExpertRange { int c, f, kh, s0, ns, G; };
-
-MOBA_DEV ExpertRange expert_range(int e, int Hq, int Hkv, const int* cu_chunk,
-                                  const int* chunk_batch, const int* cu_seqlens,
-                                  const int* filtered) {
-  ExpertRange r;
-  const int f = e / Hkv;
-  r.kh = e % Hkv;
-  r.f = f;
-  r.c = filtered[f];
-  r.s0 = cu_chunk[r.c + 1];
-  r.ns = cu_seqlens[chunk_batch[r.c] + 1] - r.s0;
-  r.G = Hq / Hkv;
-  return r;
-}
-
-// Candidates of an expert are split in blocks of kCandBlock; workgroup
-// (e, b) handles block b of expert e.  Block counts go to work[e * nbmax + b]
-// and become exclusive offsets within the expert in the scan, so the fill is
-// an ordered compaction with no atomics.
-constexpr int kCandBlock = 2048;
-
-__global__ __launch_bounds__(256) void expert_count_kernel(
-    const uint64_t* __restrict__ mask, int T, int NW, int Hq, int Hkv,
-    const int* __restrict__ cu_chunk, const int* __restrict__ chunk_batch,
-    const int* __restrict__ cu_seqlens, const int* __restrict__ filtered, int nbmax,
-    int* __restrict__ work) {
-  const int e = blockIdx.x, b = blockIdx.y;
-  ExpertRange x = expert_range(e, Hq, Hkv, cu_chunk, chunk_batch, cu_seqlens, filtered);
-  const int64_t n = (int64_t)x.G * x.ns;
-  const int64_t i1 = min(n, (int64_t)(b + 1) * kCandBlock);
-  const int mw = x.f >> 6, bit = x.f & 63;
-  int cnt = 0;
-  for (int64_t i = (int64_t)b * kCandBlock + threadIdx.x; i < i1; i += 256) {
-    const int g = (int)(i / x.ns), s = x.s0 + (int)(i % x.ns);
-    cnt += (int)((mask[((int64_t)(x.kh * x.G + g) * NW + mw) * T + s] >> bit) & 1);
-  }
+// One workgroup per expert: its block counts become exclusive offsets, and
+// their sum the expert's row count.
+__global__ __launch_bounds__(256) void expert_blocks_kernel(int* __restrict__ blk_count, int nblk,
+                                                            int Hq, int Hkv,
+                                                            int* __restrict__ counts) {
   __shared__ int part[4];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0) part[w] = cnt;
-  __syncthreads();
-  if (threadIdx.x == 0) work[(int64_t)e * nbmax + b] = part[0] + part[1] + part[2] + part[3];
+  const int e = blockIdx.x, f = e / Hkv, kh = e % Hkv, G = Hq / Hkv;
+  int* c = blk_count + ((int64_t)f * Hq + kh * G) * nblk;
+  const int n = G * nblk;
+  int run = 0;
+  for (int i0 = 0; i0 < n; i0 += 256) {
+    const int i = i0 + threadIdx.x;
+    int total;
+    const int before = block_scan_256(i < n ? c[i] : 0, total, part);
+    if (i < n) c[i] = run + before;
+    run += total;
+  }
+  if (threadIdx.x == 0) counts[e] = run;
 }
 
-// Per expert: block counts -> exclusive block offsets and the row count; then
-// exclusive scans of row counts and tile counts over the experts (one workgroup).
-__global__ __launch_bounds__(1024) void expert_scan_kernel(int* __restrict__ work, int nbmax, int E,
-                                                         int block_rows, int* __restrict__ counts,
-                                                         int* __restrict__ row_off,
-                                                         int* __restrict__ tile_off) {
-  __shared__ int wr[16], wt[16];
-  __shared__ int carry_r, carry_t;
-  if (threadIdx.x == 0) { carry_r = 0; carry_t = 0; }
-  __syncthreads();
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  for (int base = 0; base < E; base += 1024) {
-    const int e = base + threadIdx.x;
-    int r = 0;
-    if (e < E) {
-      int* wb = work + (int64_t)e * nbmax;
-      for (int b = 0; b < nbmax; ++b) { const int c = wb[b]; wb[b] = r; r += c; }
-      counts[e] = r;
-    }
-    int t = (r + block_rows - 1) / block_rows;
-    // inclusive wave scan
-    int ir = r, it = t;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      int yr = __shfl_up(ir, o, 64), yt = __shfl_up(it, o, 64);
-      if (lane >= o) { ir += yr; it += yt; }
-    }
-    if (lane == 63) { wr[w] = ir; wt[w] = it; }
-    __syncthreads();
-    int pr = carry_r, pt = carry_t;
-    for (int i = 0; i < w; ++i) { pr += wr[i]; pt += wt[i]; }
-    if (e < E) { row_off[e] = pr + ir - r; tile_off[e] = pt + it - t; }
-    __syncthreads();
-    if (threadIdx.x == 1023) { carry_r = pr + ir; carry_t = pt + it; }
-    __syncthreads();
+// Exclusive scans of row counts and tile counts over the experts (one
+// workgroup; for more experts than a fill workgroup scans by itself).
+__global__ __launch_bounds__(256) void expert_scan_kernel(const int* __restrict__ counts, int E,
+                                                          int block_rows,
+                                                          int* __restrict__ row_off,
+                                                          int* __restrict__ tile_off) {
+  __shared__ int64_t part[4];
+  int64_t run = 0;  // rows in the low half, tiles in the high half
+  for (int e0 = 0; e0 < E; e0 += 256) {
+    const int e = e0 + threadIdx.x;
+    const int r = e < E ? counts[e] : 0;
+    int64_t total;
+    const int64_t x = run + block_scan_256(
+        (int64_t)r | (int64_t)((r + block_rows - 1) / block_rows) << 32, total, part);
+    if (e < E) { row_off[e] = (int)x; tile_off[e] = (int)(x >> 32); }
+    run += total;
   }
-  if (threadIdx.x == 0) { row_off[E] = carry_r; tile_off[E] = carry_t; }
+  if (threadIdx.x == 0) { row_off[E] = (int)run; tile_off[E] = (int)(run >> 32); }
 }
 
 // Ordered compaction: rows[row_off[e] + rank] = ((s*Hq + h) << 3) | j (R <= 8).
-__global__ __launch_bounds__(256) void expert_fill_kernel(
-    const uint64_t* __restrict__ mask, int T, int NW, int Hq, int Hkv,
-    const int* __restrict__ cu_chunk, const int* __restrict__ chunk_batch,
-    const int* __restrict__ cu_seqlens, const int* __restrict__ filtered,
-    const int* __restrict__ row_off, int nbmax, const int* __restrict__ work,
-    int* __restrict__ rows) {
-  const int e = blockIdx.x, b = blockIdx.y;
-  ExpertRange x = expert_range(e, Hq, Hkv, cu_chunk, chunk_batch, cu_seqlens, filtered);
-  const int mw = x.f >> 6, bit = x.f & 63;
-  const int64_t n = (int64_t)x.G * x.ns;
-  const int64_t i0 = (int64_t)b * kCandBlock, i1 = min(n, i0 + kCandBlock);
-  if (i0 >= i1) return;
-  __shared__ int wtot[4];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int out = row_off[e] + work[(int64_t)e * nbmax + b];
-  for (int64_t base = i0; base < i1; base += 256) {
-    const int64_t i = base + threadIdx.x;
-    int slot = -1, h = 0, s = 0;
-    if (i < i1) {
-      const int g = (int)(i / x.ns);
-      s = x.s0 + (int)(i % x.ns);
-      h = x.kh * x.G + g;
-      const uint64_t* mh = mask + (int64_t)h * NW * T + s;
-      const uint64_t m = mh[(int64_t)mw * T];
-      if ((m >> bit) & 1) {
-        // slot = the selected chunks before this one (sel is ascending)
-        slot = __popcll(m & ((1ull << bit) - 1ull));
-        for (int w2 = 0; w2 < mw; ++w2) slot += __popcll(mh[(int64_t)w2 * T]);
-      }
+// Workgroup (block, h) places the picks of its 256 tokens.  With SCAN each
+// workgroup scans the experts' counts by itself (E <= kScanExperts, 8 loads
+// per thread at most) instead of waiting for a one-workgroup launch, and the
+// first one writes row_off and tile_off.
+constexpr int kScanExperts = 2048;
+
+template <bool SCAN>
+__global__ __launch_bounds__(256) void expert_fill_kernel(PackArgs a) {
+  __shared__ uint64_t bits[kPickRows * 4];
+  __shared__ int roff[SCAN ? kScanExperts : 1];
+  __shared__ int64_t part[4];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int blk = blockIdx.x, h = blockIdx.y, nblk = gridDim.x;
+  const int Hq = a.Hq, Hkv = a.Hkv, E = a.F * Hkv, block_rows = a.block_rows;
+  const int s = blk * 256 + tid, kh = h / (Hq / Hkv);
+  int fs[kMaxRemote];
+  int at[kMaxRemote];  // the block's first position within each picked expert
+  load_picks(a, s, h, fs, &at, blk, nblk);
+  if constexpr (SCAN) {
+    constexpr int PT = kScanExperts / 256;  // consecutive experts per thread
+    int n[PT];
+    int64_t mine = 0;  // rows in the low half, tiles in the high half
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+      n[i] = tid * PT + i < E ? a.counts[tid * PT + i] : 0;
+      mine += (int64_t)n[i] | (int64_t)((n[i] + block_rows - 1) / block_rows) << 32;
     }
-    const uint64_t hits = __ballot(slot >= 0);
-    const int before = __popcll(hits & ((1ull << lane) - 1ull));
-    if (lane == 0) wtot[w] = __popcll(hits);
-    __syncthreads();
-    int off = out;
-    for (int k2 = 0; k2 < w; ++k2) off += wtot[k2];
-    if (slot >= 0) rows[off + before] = (((s * Hq) + h) << 3) | slot;
-    const int tot = wtot[0] + wtot[1] + wtot[2] + wtot[3];
-    __syncthreads();
-    out += tot;
+    int64_t total, x = block_scan_256(mine, total, part);
+    const bool first = blk == 0 && h == 0;
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+      const int e = tid * PT + i;
+      if (e < E) {
+        roff[e] = (int)x;
+        if (first) { a.row_off[e] = (int)x; a.tile_off[e] = (int)(x >> 32); }
+      }
+      x += (int64_t)n[i] | (int64_t)((n[i] + block_rows - 1) / block_rows) << 32;
+    }
+    if (first && tid == 0) { a.row_off[E] = (int)total; a.tile_off[E] = (int)(total >> 32); }
+  }
+#pragma unroll
+  for (int j = 0; j < kMaxRemote; ++j) {
+    if (!SCAN && fs[j] >= 0) at[j] += a.row_off[fs[j] * Hkv + kh];
+  }
+  for (int t0 = 0; t0 < a.F; t0 += kPickRows) {
+    pick_bits(bits, fs, t0);  // its barriers order the writes of roff, too
+#pragma unroll
+    for (int j = 0; j < kMaxRemote; ++j) {
+      const int r = fs[j] - t0;
+      if (fs[j] < 0 || r < 0 || r >= kPickRows) continue;
+      const uint64_t* b = bits + 4 * r;
+      int rank = __popcll(b[w] & ((1ull << lane) - 1ull));
+      for (int i = 0; i < w; ++i) rank += __popcll(b[i]);
+      const int base = at[j] + (SCAN ? roff[fs[j] * Hkv + kh] : 0);
+      a.rows[base + rank] = ((s * Hq + h) << 3) | j;
+    }
   }
 }
 
-int64_t expert_blocks(int T, int Hq, int Hkv) {
-  return ((int64_t)(Hq / Hkv) * T + kCandBlock - 1) / kCandBlock;
+int64_t pick_blocks(int T) { return ((int64_t)T + 255) / 256; }
+
+// Offsets and rows from the block counts in a.blk.
+void launch_pack(const PackArgs& a, hipStream_t st) {
+  const int E = a.F * a.Hkv, nblk = (int)pick_blocks(a.T);
+  hipLaunchKernelGGL(expert_blocks_kernel, dim3(E), dim3(256), 0, st, a.blk, nblk, a.Hq, a.Hkv,
+                     a.counts);
+  const dim3 grid(nblk, a.Hq);
+  if (E <= kScanExperts) {
+    hipLaunchKernelGGL(expert_fill_kernel<true>, grid, dim3(256), 0, st, a);
+  } else {
+    hipLaunchKernelGGL(expert_scan_kernel, dim3(1), dim3(256), 0, st, a.counts, E, a.block_rows,
+                       a.row_off, a.tile_off);
+    hipLaunchKernelGGL(expert_fill_kernel<false>, grid, dim3(256), 0, st, a);
+  }
 }
 
 }  // namespace
@@ -447,14 +531,13 @@ extern "C" int moba_hip_chunk_means(const void* k, int dtype, int T, int Hkv, in
   return moba_launch_status("chunk_means");
 }
 
-extern "C" int moba_hip_route_prefill(const void* q, int dtype, int T, int Hq, int Hkv, int D,
-                                      const float* means, const int* cu_chunk, int nchunk,
-                                      const int* chunk_batch, const int* first_chunk, int R,
-                                      int F, int* sel, float* gate, void* stream) {
+static int route_prefill(const void* q, int dtype, int T, int Hq, int Hkv, int D,
+                         const float* means, const int* cu_chunk, int nchunk,
+                         const int* chunk_batch, const int* first_chunk, int R, int F, int* sel,
+                         float* gate, int* blk_count, hipStream_t st) {
   if (R < 1 || R > kMaxRemote) { moba_set_error("route_prefill: remote count must be in [1,8]"); return MOBA_ERR_ARG; }
   if (D % 8 || D < 8) { moba_set_error("route_prefill: head_dim must be a multiple of 8"); return MOBA_ERR_ARG; }
   if (Hq % Hkv) { moba_set_error("route_prefill: Hq must be a multiple of Hkv"); return MOBA_ERR_ARG; }
-  hipStream_t st = (hipStream_t)stream;
   if (gate) {
     const int64_t n = (int64_t)F * Hq * T;
     hipLaunchKernelGGL(fill_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, gate,
@@ -465,7 +548,7 @@ extern "C" int moba_hip_route_prefill(const void* q, int dtype, int T, int Hq, i
   const uint16_t* qp = (const uint16_t*)q;
 #define MOBA_ROUTE(DT_, DP_, DE_) \
   hipLaunchKernelGGL((route_kernel<DT_, DP_, DE_>), grid, block, 0, st, qp, T, Hq, Hkv, D, means, \
-                     cu_chunk, nchunk, chunk_batch, first_chunk, R, F, sel, gate)
+                     cu_chunk, nchunk, chunk_batch, first_chunk, R, F, sel, gate, blk_count)
 #define MOBA_ROUTE_DT(DT_) \
   if (D == 64) MOBA_ROUTE(DT_, 64, 64); else if (D < 64) MOBA_ROUTE(DT_, 64, 0); \
   else if (D == 128) MOBA_ROUTE(DT_, 128, 128); else if (D < 128) MOBA_ROUTE(DT_, 128, 0); \
@@ -480,13 +563,26 @@ extern "C" int moba_hip_route_prefill(const void* q, int dtype, int T, int Hq, i
   return moba_launch_status("route_prefill");
 }
 
-// Work ints of moba_hip_pack_experts: the selection bitmasks (2 ints per
-// 64-bit word), then the per-(expert, block) counts.
-int64_t mask_ints(int T, int Hq, int F) { return (int64_t)T * Hq * ((F + 63) / 64) * 2; }
+extern "C" int moba_hip_route_prefill(const void* q, int dtype, int T, int Hq, int Hkv, int D,
+                                      const float* means, const int* cu_chunk, int nchunk,
+                                      const int* chunk_batch, const int* first_chunk, int R,
+                                      int F, int* sel, float* gate, void* stream) {
+  return route_prefill(q, dtype, T, Hq, Hkv, D, means, cu_chunk, nchunk, chunk_batch, first_chunk,
+                       R, F, sel, gate, nullptr, (hipStream_t)stream);
+}
 
+// Work ints of the expert packing: the block counts of every (candidate, head).
 extern "C" int64_t moba_hip_pack_experts_work(int T, int Hq, int Hkv, int F) {
   if (T < 0 || Hq < 1 || Hkv < 1 || Hq % Hkv || F < 0) return -1;
-  return mask_ints(T, Hq, F) + (int64_t)F * Hkv * expert_blocks(T, Hq, Hkv);
+  return (int64_t)F * Hq * pick_blocks(T);
+}
+
+static int check_pack(int T, int Hq, int Hkv, int R, const int* work) {
+  if ((int64_t)T * Hq * R >= (1ll << 31) || (int64_t)T * Hq >= (1ll << 28)) { moba_set_error("pack_experts: T*Hq*R exceeds int32 or T*Hq exceeds 2^28"); return MOBA_ERR_ARG; }
+  if (R > 8) { moba_set_error("pack_experts: at most 8 remote chunks per query"); return MOBA_ERR_ARG; }
+  if (Hkv < 1 || Hq % Hkv) { moba_set_error("pack_experts: Hq must be a multiple of Hkv"); return MOBA_ERR_ARG; }
+  if (work == nullptr || ((uintptr_t)work & 7)) { moba_set_error("pack_experts: the work buffer (moba_hip_pack_experts_work ints, 8-byte aligned) is required"); return MOBA_ERR_ARG; }
+  return MOBA_OK;
 }
 
 extern "C" int moba_hip_pack_experts(const int* sel, int T, int Hq, int Hkv, int R,
@@ -495,24 +591,33 @@ extern "C" int moba_hip_pack_experts(const int* sel, int T, int Hq, int Hkv, int
                                      int block_rows, int* counts, int* row_off, int* tile_off,
                                      int* rows, int* work, void* stream) {
   if (F <= 0) return MOBA_OK;
-  if ((int64_t)T * Hq * R >= (1ll << 31) || (int64_t)T * Hq >= (1ll << 28)) { moba_set_error("pack_experts: T*Hq*R exceeds int32 or T*Hq exceeds 2^28"); return MOBA_ERR_ARG; }
-  if (R > 8) { moba_set_error("pack_experts: at most 8 remote chunks per query"); return MOBA_ERR_ARG; }
-  if (Hkv < 1 || Hq % Hkv) { moba_set_error("pack_experts: Hq must be a multiple of Hkv"); return MOBA_ERR_ARG; }
-  if (work == nullptr || ((uintptr_t)work & 7)) { moba_set_error("pack_experts: the work buffer (moba_hip_pack_experts_work ints, 8-byte aligned) is required"); return MOBA_ERR_ARG; }
+  if (int rc = check_pack(T, Hq, Hkv, R, work)) return rc;
+  if (T < 1) return MOBA_OK;
   hipStream_t st = (hipStream_t)stream;
-  const int E = F * Hkv;
-  const int nbmax = (int)expert_blocks(T, Hq, Hkv);
-  if (nbmax < 1) return MOBA_OK;
-  const int NW = (F + 63) / 64;
-  uint64_t* mask = reinterpret_cast<uint64_t*>(work);  // 8-byte aligned: the work buffer's start
-  int* cwork = work + mask_ints(T, Hq, F);
-  hipLaunchKernelGGL(sel_mask_kernel, dim3((unsigned)(((int64_t)T * Hq + 255) / 256)), dim3(256),
-                     0, st, sel, T, Hq, R, chunk_batch, NW, mask);
-  hipLaunchKernelGGL(expert_count_kernel, dim3(E, nbmax), dim3(256), 0, st, mask, T, NW, Hq, Hkv,
-                     cu_chunk, chunk_batch, cu_seqlens, filtered, nbmax, cwork);
-  hipLaunchKernelGGL(expert_scan_kernel, dim3(1), dim3(1024), 0, st, cwork, nbmax, E, block_rows,
-                     counts, row_off, tile_off);
-  hipLaunchKernelGGL(expert_fill_kernel, dim3(E, nbmax), dim3(256), 0, st, mask, T, NW, Hq, Hkv,
-                     cu_chunk, chunk_batch, cu_seqlens, filtered, row_off, nbmax, cwork, rows);
+  const PackArgs a = {sel, T, Hq, Hkv, R, cu_chunk, chunk_batch, cu_seqlens, filtered, F,
+                      block_rows, counts, row_off, tile_off, rows, work};
+  hipLaunchKernelGGL(pick_count_kernel, dim3((unsigned)pick_blocks(T), Hq), dim3(256), 0, st, a);
+  launch_pack(a, st);
   return moba_launch_status("pack_experts");
+}
+
+extern "C" int moba_hip_prefill_route(const void* q, const void* k, int dtype, int T, int Hq,
+                                      int Hkv, int D, const int* chunk_start, int chunk,
+                                      int precision, const int* cu_chunk, int nchunk,
+                                      const int* chunk_batch, const int* first_chunk,
+                                      const int* cu_seqlens, const int* filtered, int R, int F,
+                                      int block_rows, float* means, int* sel, float* gate,
+                                      int* counts, int* row_off, int* tile_off, int* rows,
+                                      int* work, void* stream) {
+  if (F <= 0) return MOBA_OK;
+  if (Hkv < 1 || Hq < 1) { moba_set_error("prefill_route: bad head counts"); return MOBA_ERR_ARG; }
+  if (int rc = check_pack(T, Hq, Hkv, R, work)) return rc;
+  if (int rc = moba_hip_chunk_means(k, dtype, T, Hkv, D, chunk_start, F, chunk, precision, means,
+                                    stream)) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  if (int rc = route_prefill(q, dtype, T, Hq, Hkv, D, means, cu_chunk, nchunk, chunk_batch,
+                             first_chunk, R, F, sel, gate, work, st)) return rc;
+  launch_pack({sel, T, Hq, Hkv, R, cu_chunk, chunk_batch, cu_seqlens, filtered, F, block_rows,
+               counts, row_off, tile_off, rows, work}, st);
+  return moba_launch_status("prefill_route");
 }

@@ -233,16 +233,12 @@ def route(plan: PrefillPlan, q, k, precision: int, want_gate=False):
     gate = torch.empty((F, hq, T), dtype=torch.float32, device=dev) if want_gate else None
     work = torch.empty(max(1, _lib.load().moba_hip_pack_experts_work(T, hq, plan.hkv, F)),
                        dtype=torch.int32, device=dev)
-    _lib.call("moba_hip_chunk_means", k.data_ptr(), code, T, plan.hkv, d,
-              plan.ptr("chunk_start"), F, plan.chunk, precision, r.means.data_ptr(), st)
-    _lib.call("moba_hip_route_prefill", q.data_ptr(), code, T, hq, plan.hkv, d,
-              r.means.data_ptr(), plan.ptr("cu_chunk"), len(plan.chunk_batch),
-              plan.ptr("chunk_batch"), plan.ptr("first_chunk"), R, F, r.sel.data_ptr(),
-              _lib.ptr(gate), st)
-    _lib.call("moba_hip_pack_experts", r.sel.data_ptr(), T, hq, plan.hkv, R,
-              plan.ptr("cu_chunk"), plan.ptr("chunk_batch"), plan.ptr("cu_seqlens"),
-              plan.ptr("filtered"), F, plan.block_rows, r.counts.data_ptr(), r.row_off.data_ptr(),
-              r.tile_off.data_ptr(), r.rows.data_ptr(), work.data_ptr(), st)
+    _lib.call("moba_hip_prefill_route", q.data_ptr(), k.data_ptr(), code, T, hq, plan.hkv, d,
+              plan.ptr("chunk_start"), plan.chunk, precision, plan.ptr("cu_chunk"),
+              len(plan.chunk_batch), plan.ptr("chunk_batch"), plan.ptr("first_chunk"),
+              plan.ptr("cu_seqlens"), plan.ptr("filtered"), R, F, plan.block_rows,
+              r.means.data_ptr(), r.sel.data_ptr(), _lib.ptr(gate), r.counts.data_ptr(),
+              r.row_off.data_ptr(), r.tile_off.data_ptr(), r.rows.data_ptr(), work.data_ptr(), st)
     return (r, gate) if want_gate else r
 
 

@@ -391,3 +391,49 @@ def test_route_hook_matches_oracle(cuda_device, hq, hkv, lens, chunk, topk):
     assert want.any() and not want.all()
     moba_hip.run_impl("opt_hip", q, k, v, cu, ml, cfg)   # unset: not called again
     assert len(calls) == 1
+
+
+@pytest.mark.parametrize("hq,hkv,lens,chunk,topk", [
+    (4, 2, (255, 256, 257, 1), 64, 3),    # blocks of 256 tokens that end with, before and after one
+    (6, 3, (17, 1, 90), 8, 9),            # one block, several sequences in it
+    (2, 1, (4200,), 16, 4),               # 262 candidates: more than one tile of pick bits
+    (24, 12, (3001,), 16, 3),             # 2244 experts: scanned in their own launch
+])
+def test_expert_lists(cuda_device, hq, hkv, lens, chunk, topk):
+    """The packing of the one-call routing and of moba_hip_pack_experts (given
+    the selection alone) against the lists that the selection spells out."""
+    from moba_hip.ops import _lib
+    from moba_hip.ops import prefill as P
+    q, k, v, cu, ml, _ = prefill_inputs(hq, hkv, 64, lens, torch.bfloat16, seed=23)
+    plan, rt, _ = _gpu_route(q, k, cu, {"chunk_size": chunk, "topk": topk})
+    T, F, R, E = q.shape[0], plan.num_filtered, plan.remote, plan.num_experts
+    sel, G = rt.sel.cpu().numpy(), hq // hkv
+    rows = [[] for _ in range(E)]
+    fidx = {c: f for f, c in enumerate(plan.filtered)}
+    for h in range(hq):
+        for s in range(T):
+            for j in range(R):
+                if sel[s, h, j] >= 0:
+                    rows[fidx[sel[s, h, j]] * hkv + h // G].append((s * hq + h) << 3 | j)
+    counts = np.array([len(r) for r in rows])
+    tiles = -(-counts // plan.block_rows)
+    other = P.RouteResult()
+    for name in ("counts", "row_off", "tile_off", "rows"):
+        setattr(other, name, torch.full_like(getattr(rt, name), -7))
+    work = torch.empty(_lib.load().moba_hip_pack_experts_work(T, hq, hkv, F), dtype=torch.int32,
+                       device="cuda")
+    # entries that are not candidates of their token (its own chunk) are left out
+    given = rt.sel.clone()
+    own = torch.tensor(np.searchsorted(plan.cu_chunk, np.arange(T), "right") - 1, device="cuda",
+                       dtype=torch.int32)[:, None, None].expand_as(given)
+    given = torch.where(given < 0, own, given)
+    _lib.call("moba_hip_pack_experts", given.data_ptr(), T, hq, hkv, R, plan.ptr("cu_chunk"),
+              plan.ptr("chunk_batch"), plan.ptr("cu_seqlens"), plan.ptr("filtered"), F,
+              plan.block_rows, other.counts.data_ptr(), other.row_off.data_ptr(),
+              other.tile_off.data_ptr(), other.rows.data_ptr(), work.data_ptr(),
+              _lib.stream_of(q.device))
+    for r in (rt, other):
+        np.testing.assert_array_equal(r.counts.cpu().numpy(), counts)
+        np.testing.assert_array_equal(r.row_off.cpu().numpy(), np.r_[0, counts.cumsum()])
+        np.testing.assert_array_equal(r.tile_off.cpu().numpy(), np.r_[0, tiles.cumsum()])
+        np.testing.assert_array_equal(r.rows.cpu().numpy()[:counts.sum()], np.concatenate(rows))
