@@ -82,14 +82,17 @@ int64_t moba_hip_pack_experts_work(int T, int Hq, int Hkv, int F);
 
 /* moba_hip_chunk_means, moba_hip_route_prefill and moba_hip_pack_experts in
  * one call (the same arguments and results): the gate kernel counts the picks
- * of its blocks while it has them, so the packing reads them once. */
+ * of its blocks while it has them, so the packing reads them once.  tiles
+ * (nullable; 16-byte aligned) [n_tiles][4] int32 receives the work of the
+ * remote kernels, workgroup by workgroup, for the _tiles entries below:
+ * n_tiles = their max_remote_tiles rounded up to a multiple of 8. */
 int moba_hip_prefill_route(const void* q, const void* k, int dtype, int T, int Hq, int Hkv, int D,
                            const int* chunk_start, int chunk, int precision,
                            const int* cu_chunk, int nchunk, const int* chunk_batch,
                            const int* first_chunk, const int* cu_seqlens, const int* filtered,
                            int R, int F, int block_rows, float* means, int* sel, float* gate,
-                           int* counts, int* row_off, int* tile_off, int* rows, int* work,
-                           void* stream);
+                           int* counts, int* row_off, int* tile_off, int* rows, int* tiles,
+                           int n_tiles, int* work, void* stream);
 
 /* Query rows per prefill tile for head dim D (-1 for an unsupported D): the
  * block_rows of moba_hip_pack_experts and the row step of the self tiles
@@ -117,6 +120,16 @@ int moba_hip_prefill_fwd(const void* q, const void* k, const void* v, int dtype,
                          const int* tile_off, const int* row_off, const int* counts,
                          const int* rows, int max_remote_tiles, void* part_o, float* part_ml,
                          void* out, float* lse, void* stream);
+
+/* The same with the tiles that moba_hip_prefill_route wrote: a remote
+ * workgroup starts from its entry instead of a search of tile_off. */
+int moba_hip_prefill_fwd_tiles(const void* q, const void* k, const void* v, int dtype, int T,
+                               int Hq, int Hkv, int D, float scale, const int* cu_chunk,
+                               const int* self_tiles, int n_self_tiles, const int* sel, int R,
+                               const int* filtered, int E, const int* tile_off,
+                               const int* row_off, const int* counts, const int* rows,
+                               const int* tiles, int max_remote_tiles, void* part_o,
+                               float* part_ml, void* out, float* lse, void* stream);
 
 /* Backward of moba_hip_prefill_fwd with the GLOBAL O and LSE.
  * Replaces OptMixedAttention.backward (src/moba_opt/mixed_attention.py:141-225):
@@ -151,6 +164,18 @@ int moba_hip_prefill_bwd(const void* q, const void* k, const void* v, const void
                          int max_remote_tiles, float* delta, void* part_dq, void* dq, void* dk,
                          void* dv, int parts, int kv_splits, float* part_dkv, void* pack,
                          void* stream);
+
+/* The same with the tiles that moba_hip_prefill_route wrote. */
+int moba_hip_prefill_bwd_tiles(const void* q, const void* k, const void* v, const void* out,
+                               const void* dout, const float* lse, int dtype, int T, int Hq,
+                               int Hkv, int D, float scale, const int* cu_chunk,
+                               const int* self_tiles, int n_self_tiles, const int* kv_tiles,
+                               int n_kv_tiles, const int* sel, int R, const int* filtered, int E,
+                               const int* tile_off, const int* row_off, const int* counts,
+                               const int* rows, const int* tiles, int max_remote_tiles,
+                               float* delta, void* part_dq, void* dq, void* dk, void* dv,
+                               int parts, int kv_splits, float* part_dkv, void* pack,
+                               void* stream);
 
 /* Bytes of the row-split workspace moba_hip_prefill_bwd needs for kv_splits
  * > 1 (0 for kv_splits < 2 or bad arguments).  No counterpart in the

@@ -76,32 +76,21 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
 
   int s[QB], h[QB], slot[QB];
   int pidx[QB];  // packed index of an expert row (row_off order)
+  int packed[QB];
   bool valid[QB];
   int kh, k_lo, k_hi, s_wave0 = 0;
   if constexpr (REMOTE) {
-    const int t = xcd_contiguous(blockIdx.x, a.tile_off[a.E]);
-    if (t < 0) return;
-    int lo = 0, hi = a.E - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (a.tile_off[mid] <= t) lo = mid; else hi = mid - 1;
-    }
-    const int e = lo;
-    kh = e % a.Hkv;
-    const int c = a.filtered[e / a.Hkv];
-    k_lo = a.cu_chunk[c];
-    k_hi = a.cu_chunk[c + 1];
-    const int cnt = a.counts[e], base = a.row_off[e];
+    const ExpertTile x = expert_tile<128 * QB>(a);
+    if (x.rows == 0) return;
+    kh = x.kh;
+    k_lo = x.k_lo;
+    k_hi = x.k_hi;
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
-      const int local = (t - a.tile_off[e]) * (128 * QB) + wave * (32 * QB) + qb * 32 + qi;
-      valid[qb] = local < cnt;
-      pidx[qb] = base + local;
-      const int packed = valid[qb] ? a.rows[base + local] : 0;  // (row << 3) | j
-      const int sh = packed >> 3;
-      slot[qb] = sh * a.R + (packed & 7);
-      s[qb] = sh / a.Hq;
-      h[qb] = sh % a.Hq;
+      const int local = wave * (32 * QB) + qb * 32 + qi;
+      valid[qb] = local < x.rows;
+      pidx[qb] = x.row0 + local;
+      packed[qb] = a.rows[x.row0 + min(local, x.rows - 1)];  // (row << 3) | j
     }
   } else {
     // 1-D grid over (tile, q head within the kv group), tiles in the
@@ -127,47 +116,6 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
       if (!valid[qb]) s[qb] = k_hi - 1;
     }
   }
-  u16x8_t qf[QB][NKS], gf[QB][NKS];
-  float lse2[QB], lk[QB], dl[QB];
-#pragma unroll
-  for (int qb = 0; qb < QB; ++qb) {
-    const int64_t row = (int64_t)s[qb] * a.Hq + h[qb];
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      const int d = ks * 16 + hh * 8;
-      const bool ok = valid[qb] && d < D;
-      qf[qb][ks] = ok ? ld8(a.q + row * D + d) : zero8();
-      gf[qb][ks] = ok ? ld8(a.dout + row * D + d) : zero8();
-    }
-    const float lr = valid[qb] ? a.lse[row] : INFINITY;
-    lse2[qb] = lr * kLog2e;
-    lk[qb] = lr / a.scale;
-    dl[qb] = valid[qb] ? a.delta[row] : 0.0f;
-  }
-  if constexpr (REMOTE && DP <= 128) {
-    // The key-major dK/dV kernel reads the expert rows packed contiguously in
-    // row_off order; this kernel holds exactly those rows, so it writes the
-    // packed q / dO / lse_k / delta (the values delta_kernel and the loads above
-    // produce) instead of a separate gather pass.
-#pragma unroll
-    for (int qb = 0; qb < QB; ++qb) {
-      if (!valid[qb]) continue;
-      const int64_t m = pidx[qb];
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        const int d = ks * 16 + hh * 8;
-        if (d < D) {
-          st8(a.pack_q + m * D + d, qf[qb][ks]);
-          st8(a.pack_g + m * D + d, gf[qb][ks]);
-        }
-      }
-      if (hh == 0) {
-        a.pack_lse_k[m] = lk[qb];
-        a.pack_delta[m] = dl[qb];
-      }
-    }
-  }
-
   const int wave_s = __builtin_amdgcn_readfirstlane(wave);
   // Lane l of wave w loads blocks j = (n * 4 + w) * 64 + l: row j / NB,
   // physical block j % NB.  The row advances by 256 / NB per n, a multiple of
@@ -211,6 +159,66 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
     }
     __syncthreads();
   }
+  // The first K / V tile goes out before the query rows: an expert's rows
+  // wait for their row list, the tile only for the workgroup's entry (above
+  // 128 dims the rows come first and each load is guarded: otherwise the
+  // kernel spills 325 registers).  Rows past the tile's end load the last
+  // row's data and are never written.
+  constexpr bool TILE_FIRST = DP <= 128;
+  if constexpr (TILE_FIRST) dma(K0, V0, 0);
+  u16x8_t qf[QB][NKS], gf[QB][NKS];
+  float lse2[QB], lk[QB], dl[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    if constexpr (REMOTE) {
+      const int sh = packed[qb] >> 3;
+      slot[qb] = sh * a.R + (packed[qb] & 7);
+      s[qb] = sh / a.Hq;
+      h[qb] = sh % a.Hq;
+    }
+    const int64_t row = (int64_t)s[qb] * a.Hq + h[qb];
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      const int d = ks * 16 + hh * 8, dc = d < D ? d : 0;
+      if constexpr (TILE_FIRST) {
+        const u16x8_t xq = ld8(a.q + row * D + dc), xg = ld8(a.dout + row * D + dc);
+        qf[qb][ks] = d < D ? xq : zero8();
+        gf[qb][ks] = d < D ? xg : zero8();
+      } else {
+        qf[qb][ks] = valid[qb] && d < D ? ld8(a.q + row * D + d) : zero8();
+        gf[qb][ks] = valid[qb] && d < D ? ld8(a.dout + row * D + d) : zero8();
+      }
+    }
+    const float lr = a.lse[row];
+    lse2[qb] = lr * kLog2e;
+    lk[qb] = lr / a.scale;
+    dl[qb] = a.delta[row];
+  }
+  if constexpr (REMOTE && DP <= 128) {
+    // The key-major dK/dV kernel reads the expert rows packed contiguously in
+    // row_off order; this kernel holds exactly those rows, so it writes the
+    // packed q / dO / lse_k / delta (the values delta_kernel and the loads above
+    // produce) instead of a separate gather pass.
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      if (!valid[qb]) continue;
+      const int64_t m = pidx[qb];
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) {
+        const int d = ks * 16 + hh * 8;
+        if (d < D) {
+          st8(a.pack_q + m * D + d, qf[qb][ks]);
+          st8(a.pack_g + m * D + d, gf[qb][ks]);
+        }
+      }
+      if (hh == 0) {
+        a.pack_lse_k[m] = lk[qb];
+        a.pack_delta[m] = dl[qb];
+      }
+    }
+  }
+
+  if constexpr (!TILE_FIRST) dma(K0, V0, 0);
   const uint32_t kbase0 = swz_b128_base<DP>(lane);
   const uint32_t trb0 = swz_tr_base<DP>(lane, 0), trb1 = swz_tr_base<DP>(lane, 1);
 
@@ -355,7 +363,6 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
     const bool need_mask = (kt0 + kBN > k_hi) || (!REMOTE && kt0 + kBN - 1 > s_wave0);
     if (need_mask) tile(Kb, Vb, it, std::true_type{}); else tile(Kb, Vb, it, std::false_type{});
   };
-  dma(K0, V0, 0);
   stage_sync();
   for (int it = 0; it < ntiles; it += 2) {
     if (it + 1 < ntiles) dma(K1, V1, it + 1);
@@ -973,13 +980,14 @@ extern "C" int64_t moba_hip_prefill_bwd_work(int n_kv_tiles, int kv_splits, int 
          (int64_t)n_kv_tiles * kv_splits * kv_slot_floats(D) * 4;
 }
 
-extern "C" int moba_hip_prefill_bwd(const void* q, const void* k, const void* v, const void* out,
+extern "C" int moba_hip_prefill_bwd_tiles(const void* q, const void* k, const void* v, const void* out,
                                     const void* dout, const float* lse, int dtype, int T, int Hq,
                                     int Hkv, int D, float scale, const int* cu_chunk,
                                     const int* self_tiles, int n_self_tiles, const int* kv_tiles,
                                     int n_kv_tiles, const int* sel, int R, const int* filtered,
                                     int E, const int* tile_off, const int* row_off,
-                                    const int* counts, const int* rows, int max_remote_tiles,
+                                    const int* counts, const int* rows, const int* tiles,
+                                    int max_remote_tiles,
                                     float* delta, void* part_dq, void* dq, void* dk, void* dv,
                                     int parts, int kv_splits, float* part_dkv, void* pack,
                                     void* stream) {
@@ -1002,6 +1010,7 @@ extern "C" int moba_hip_prefill_bwd(const void* q, const void* k, const void* v,
   a.n_self_wg = n_self_tiles * (Hq / Hkv);
   a.sel = sel; a.R = R; a.filtered = filtered; a.E = E;
   a.tile_off = tile_off; a.row_off = row_off; a.counts = counts; a.rows = rows;
+  a.tiles = (const int4*)tiles;
   a.delta = delta; a.part_dq = (uint16_t*)part_dq; a.kv_splits = kv_splits;
   a.kv_sched = a.kv_seg = nullptr; a.part_dkv = nullptr;
   if (kv_splits > 1) {  // workspace: schedule, tile slots, then the partial slots
@@ -1023,4 +1032,21 @@ extern "C" int moba_hip_prefill_bwd(const void* q, const void* k, const void* v,
   const int mr = R > 0 ? max_remote_tiles : 0;
   return dtype == 0 ? dispatch_bwd<0>(a, n_self_tiles, n_kv_tiles, mr, parts, st)
                     : dispatch_bwd<1>(a, n_self_tiles, n_kv_tiles, mr, parts, st);
+}
+
+extern "C" int moba_hip_prefill_bwd(const void* q, const void* k, const void* v, const void* out,
+                                    const void* dout, const float* lse, int dtype, int T, int Hq,
+                                    int Hkv, int D, float scale, const int* cu_chunk,
+                                    const int* self_tiles, int n_self_tiles, const int* kv_tiles,
+                                    int n_kv_tiles, const int* sel, int R, const int* filtered,
+                                    int E, const int* tile_off, const int* row_off,
+                                    const int* counts, const int* rows, int max_remote_tiles,
+                                    float* delta, void* part_dq, void* dq, void* dk, void* dv,
+                                    int parts, int kv_splits, float* part_dkv, void* pack,
+                                    void* stream) {
+  return moba_hip_prefill_bwd_tiles(q, k, v, out, dout, lse, dtype, T, Hq, Hkv, D, scale, cu_chunk,
+                                    self_tiles, n_self_tiles, kv_tiles, n_kv_tiles, sel, R,
+                                    filtered, E, tile_off, row_off, counts, rows, nullptr,
+                                    max_remote_tiles, delta, part_dq, dq, dk, dv, parts, kv_splits,
+                                    part_dkv, pack, stream);
 }

@@ -53,6 +53,7 @@ struct FwdArgs {
   const int* row_off;
   const int* counts;
   const int* rows;
+  const int4* tiles;    // remote tile of every workgroup, or null: searched
   uint16_t* part_o;     // remote partial outputs, input dtype
   float* part_ml;
   uint16_t* out;
@@ -82,31 +83,20 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
   const int D = a.D;
 
   int s[QB], h[QB], slot[QB];
+  int packed[QB];
   bool valid[QB];
   int kh, k_lo, k_hi, s_wave0 = 0;
   if constexpr (REMOTE) {
-    const int t = xcd_contiguous(blockIdx.x, a.tile_off[a.E]);
-    if (t < 0) return;
-    int lo = 0, hi = a.E - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (a.tile_off[mid] <= t) lo = mid; else hi = mid - 1;
-    }
-    const int e = lo;
-    kh = e % a.Hkv;
-    const int c = a.filtered[e / a.Hkv];
-    k_lo = a.cu_chunk[c];
-    k_hi = a.cu_chunk[c + 1];
-    const int cnt = a.counts[e], base = a.row_off[e];
+    const ExpertTile x = expert_tile<128 * QB>(a);
+    if (x.rows == 0) return;
+    kh = x.kh;
+    k_lo = x.k_lo;
+    k_hi = x.k_hi;
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
-      const int local = (t - a.tile_off[e]) * (128 * QB) + wave * (32 * QB) + qb * 32 + qi;
-      valid[qb] = local < cnt;
-      const int packed = valid[qb] ? a.rows[base + local] : 0;  // (row << 3) | j
-      const int sh = packed >> 3;
-      slot[qb] = sh * a.R + (packed & 7);
-      s[qb] = sh / a.Hq;
-      h[qb] = sh % a.Hq;
+      const int local = wave * (32 * QB) + qb * 32 + qi;
+      valid[qb] = local < x.rows;
+      packed[qb] = a.rows[x.row0 + min(local, x.rows - 1)];  // (row << 3) | j
     }
   } else {
     // 1-D grid over (tile, q head within the kv group), tiles in the
@@ -130,17 +120,6 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
       s[qb] = s_wave0 + qb * 32 + qi;
       valid[qb] = s[qb] < c_end;
       if (!valid[qb]) s[qb] = k_hi - 1;
-    }
-  }
-
-  u16x8_t qf[QB][NKS];
-#pragma unroll
-  for (int qb = 0; qb < QB; ++qb) {
-    const int64_t qrow = ((int64_t)s[qb] * a.Hq + h[qb]) * D;
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      const int d = ks * 16 + hh * 8;
-      qf[qb][ks] = (valid[qb] && d < D) ? ld8(a.q + qrow + d) : zero8();
     }
   }
 
@@ -192,6 +171,28 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
       st8(K1 + j * 8, zero8()); st8(V1 + j * 8, zero8());
     }
     __syncthreads();
+  }
+
+  // The first K / V tile goes out before the query rows: an expert's rows
+  // wait for their row list, the tile only for the workgroup's entry.  Rows
+  // past the tile's end load the last row's data and are never written.
+  dma(K0, V0, 0);
+  u16x8_t qf[QB][NKS];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    if constexpr (REMOTE) {
+      const int sh = packed[qb] >> 3;
+      slot[qb] = sh * a.R + (packed[qb] & 7);
+      s[qb] = sh / a.Hq;
+      h[qb] = sh % a.Hq;
+    }
+    const int64_t qrow = ((int64_t)s[qb] * a.Hq + h[qb]) * D;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      const int d = ks * 16 + hh * 8;
+      const u16x8_t x = ld8(a.q + qrow + (d < D ? d : 0));
+      qf[qb][ks] = d < D ? x : zero8();
+    }
   }
 
   f32x16_t oacc[QB][NDB];
@@ -306,7 +307,6 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
     const bool need_mask = (kt0 + kBN > k_hi) || (!REMOTE && kt0 + kBN - 1 > s_wave0);
     if (need_mask) tile(Kb, Vb, it, std::true_type{}); else tile(Kb, Vb, it, std::false_type{});
   };
-  dma(K0, V0, 0);
   stage_sync();
   for (int it = 0; it < ntiles; it += 2) {
     if (it + 1 < ntiles) dma(K1, V1, it + 1);
@@ -442,13 +442,14 @@ extern "C" int moba_hip_prefill_rows(int D) {
   return 128 * attn_qb<256>();
 }
 
-extern "C" int moba_hip_prefill_fwd(const void* q, const void* k, const void* v, int dtype, int T,
-                                    int Hq, int Hkv, int D, float scale, const int* cu_chunk,
-                                    const int* self_tiles, int n_self_tiles, const int* sel, int R,
-                                    const int* filtered, int E, const int* tile_off,
-                                    const int* row_off, const int* counts, const int* rows,
-                                    int max_remote_tiles, void* part_o, float* part_ml,
-                                    void* out, float* lse, void* stream) {
+extern "C" int moba_hip_prefill_fwd_tiles(const void* q, const void* k, const void* v, int dtype,
+                                          int T, int Hq, int Hkv, int D, float scale,
+                                          const int* cu_chunk, const int* self_tiles,
+                                          int n_self_tiles, const int* sel, int R,
+                                          const int* filtered, int E, const int* tile_off,
+                                          const int* row_off, const int* counts, const int* rows,
+                                          const int* tiles, int max_remote_tiles, void* part_o,
+                                          float* part_ml, void* out, float* lse, void* stream) {
   if (dtype != 0 && dtype != 1) { moba_set_error("prefill_fwd: dtype must be 0 (bf16) or 1 (fp16)"); return MOBA_ERR_ARG; }
   if (D < 8 || D > 256 || D % 8) { moba_set_error("prefill_fwd: head_dim must be a multiple of 8 in [8,256]"); return MOBA_ERR_ARG; }
   if (Hq < 1 || Hkv < 1 || Hq % Hkv) { moba_set_error("prefill_fwd: Hq must be a positive multiple of Hkv"); return MOBA_ERR_ARG; }
@@ -461,9 +462,23 @@ extern "C" int moba_hip_prefill_fwd(const void* q, const void* k, const void* v,
   a.cu_chunk = cu_chunk; a.self_tiles = self_tiles; a.n_self_wg = n_self_tiles * (Hq / Hkv);
   a.sel = sel; a.R = R; a.filtered = filtered; a.E = E;
   a.tile_off = tile_off; a.row_off = row_off; a.counts = counts; a.rows = rows;
+  a.tiles = (const int4*)tiles;
   a.part_o = (uint16_t*)part_o; a.part_ml = part_ml;
   a.out = (uint16_t*)out; a.lse = lse;
   hipStream_t st = (hipStream_t)stream;
   return dtype == 0 ? dispatch_fwd<0>(a, n_self_tiles, R > 0 ? max_remote_tiles : 0, st)
                     : dispatch_fwd<1>(a, n_self_tiles, R > 0 ? max_remote_tiles : 0, st);
+}
+
+extern "C" int moba_hip_prefill_fwd(const void* q, const void* k, const void* v, int dtype, int T,
+                                    int Hq, int Hkv, int D, float scale, const int* cu_chunk,
+                                    const int* self_tiles, int n_self_tiles, const int* sel, int R,
+                                    const int* filtered, int E, const int* tile_off,
+                                    const int* row_off, const int* counts, const int* rows,
+                                    int max_remote_tiles, void* part_o, float* part_ml,
+                                    void* out, float* lse, void* stream) {
+  return moba_hip_prefill_fwd_tiles(q, k, v, dtype, T, Hq, Hkv, D, scale, cu_chunk, self_tiles,
+                                    n_self_tiles, sel, R, filtered, E, tile_off, row_off, counts,
+                                    rows, nullptr, max_remote_tiles, part_o, part_ml, out, lse,
+                                    stream);
 }

@@ -27,6 +27,7 @@ struct BwdArgs {
   const int* row_off;
   const int* counts;
   const int* rows;
+  const int4* tiles;  // remote tile of every workgroup, or null: searched
   // delta and lse_k are one allocation, lse_k = delta + T*Hq (the key-major
   // kernels fetch both of a row with one load); likewise pack_delta =
   // pack_lse_k + pack_rows

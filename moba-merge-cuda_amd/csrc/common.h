@@ -294,6 +294,27 @@ MOBA_DEV int xcd_contiguous(int L, int total) {
   return (i < per && t < total) ? t : -1;
 }
 
+// The tile of expert rows of a remote workgroup (rows 0: none): the entry of
+// the list that the packing wrote, or, without one, the expert that tile
+// xcd_contiguous(blockIdx.x) of tile_off belongs to.  Args: FwdArgs or BwdArgs.
+struct ExpertTile { int kh, k_lo, k_hi, row0, rows; };
+template <int ROWS, typename Args> MOBA_DEV ExpertTile expert_tile(const Args& a) {
+  if (a.tiles != nullptr) {
+    const int4 d = a.tiles[blockIdx.x];
+    return {d.w >> 9, d.x, d.x + d.y, d.z, d.w & 511};
+  }
+  const int t = xcd_contiguous(blockIdx.x, a.tile_off[a.E]);
+  if (t < 0) return {0, 0, 0, 0, 0};
+  int lo = 0, hi = a.E - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (a.tile_off[mid] <= t) lo = mid; else hi = mid - 1;
+  }
+  const int c = a.filtered[lo / a.Hkv], first = (t - a.tile_off[lo]) * ROWS;
+  return {lo % a.Hkv, a.cu_chunk[c], a.cu_chunk[c + 1], a.row_off[lo] + first,
+          min(ROWS, a.counts[lo] - first)};
+}
+
 // Wave issue priority (0 or 1): a wave in an MFMA-heavy phase is set ahead of
 // a wave in an element-wise phase on the same SIMD, which keeps the matrix
 // unit fed.  No scheduling fences: the compiler keeps s_setprio in order with

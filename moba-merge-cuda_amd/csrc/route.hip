@@ -313,6 +313,8 @@ struct PackArgs {
   const int *cu_chunk, *chunk_batch, *cu_seqlens, *filtered;
   int F, block_rows;
   int *counts, *row_off, *tile_off, *rows, *blk;
+  int4* tiles;   // remote tile of every workgroup (ExpertTile), or null
+  int n_tiles;   // entries of tiles
 };
 
 // Filtered index of each pick of (s, h); -1 for none and for an entry that is
@@ -419,6 +421,32 @@ __global__ __launch_bounds__(256) void expert_scan_kernel(const int* __restrict_
   if (threadIdx.x == 0) { row_off[E] = (int)run; tile_off[E] = (int)(run >> 32); }
 }
 
+// The remote kernels' work, workgroup by workgroup: entry L is the tile that
+// xcd_contiguous gives workgroup L, as {first key, keys, first row of the row
+// list, kv head << 9 | rows}; 0 rows where there is none.  One 16-byte load
+// then starts a workgroup that would otherwise search tile_off for its expert
+// and follow the expert to its chunk (11 dependent loads at 504 experts): at
+// T 32768, 8 heads, chunk 512 the remote dQ kernel went from 494 to 444 us and
+// the remote forward from 325 to 317, with the first K / V tile on its way
+// before the query rows.
+// Workgroup w of nwg fills in the experts w, w + nwg, ... and its share of the
+// empty entries.
+MOBA_DEV void write_tiles(const PackArgs& a, int e, int row0, int tile0, int total) {
+  const int per = (total + 7) >> 3, n = a.counts[e], c = a.filtered[e / a.Hkv];
+  const int k_lo = a.cu_chunk[c], nk = a.cu_chunk[c + 1] - k_lo, kh = e % a.Hkv;
+  for (int i = threadIdx.x; i * a.block_rows < n; i += 256) {
+    const int t = tile0 + i, rows = min(a.block_rows, n - i * a.block_rows);
+    const int4 v = {k_lo, nk, row0 + i * a.block_rows, kh << 9 | rows};
+    const int L = (t % per) * 8 + t / per;
+    if (L < a.n_tiles) a.tiles[L] = v;
+  }
+}
+MOBA_DEV void clear_tiles(const PackArgs& a, int w, int nwg, int total) {
+  const int per = (total + 7) >> 3;
+  for (int L = w * 256 + threadIdx.x; L < a.n_tiles; L += nwg * 256)
+    if ((L >> 3) >= per || (L & 7) * per + (L >> 3) >= total) a.tiles[L] = {0, 0, 0, 0};
+}
+
 // Ordered compaction: rows[row_off[e] + rank] = ((s*Hq + h) << 3) | j (R <= 8).
 // Workgroup (block, h) places the picks of its 256 tokens.  With SCAN each
 // workgroup scans the experts' counts by itself (E <= kScanExperts, 8 loads
@@ -429,7 +457,7 @@ constexpr int kScanExperts = 2048;
 template <bool SCAN>
 __global__ __launch_bounds__(256) void expert_fill_kernel(PackArgs a) {
   __shared__ uint64_t bits[kPickRows * 4];
-  __shared__ int roff[SCAN ? kScanExperts : 1];
+  __shared__ int64_t off[SCAN ? kScanExperts : 1];  // rows in the low half, tiles in the high half
   __shared__ int64_t part[4];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int blk = blockIdx.x, h = blockIdx.y, nblk = gridDim.x;
@@ -438,22 +466,23 @@ __global__ __launch_bounds__(256) void expert_fill_kernel(PackArgs a) {
   int fs[kMaxRemote];
   int at[kMaxRemote];  // the block's first position within each picked expert
   load_picks(a, s, h, fs, &at, blk, nblk);
+  int64_t total = 0;
   if constexpr (SCAN) {
     constexpr int PT = kScanExperts / 256;  // consecutive experts per thread
     int n[PT];
-    int64_t mine = 0;  // rows in the low half, tiles in the high half
+    int64_t mine = 0;
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
       n[i] = tid * PT + i < E ? a.counts[tid * PT + i] : 0;
       mine += (int64_t)n[i] | (int64_t)((n[i] + block_rows - 1) / block_rows) << 32;
     }
-    int64_t total, x = block_scan_256(mine, total, part);
+    int64_t x = block_scan_256(mine, total, part);
     const bool first = blk == 0 && h == 0;
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
       const int e = tid * PT + i;
       if (e < E) {
-        roff[e] = (int)x;
+        off[e] = x;
         if (first) { a.row_off[e] = (int)x; a.tile_off[e] = (int)(x >> 32); }
       }
       x += (int64_t)n[i] | (int64_t)((n[i] + block_rows - 1) / block_rows) << 32;
@@ -465,7 +494,7 @@ __global__ __launch_bounds__(256) void expert_fill_kernel(PackArgs a) {
     if (!SCAN && fs[j] >= 0) at[j] += a.row_off[fs[j] * Hkv + kh];
   }
   for (int t0 = 0; t0 < a.F; t0 += kPickRows) {
-    pick_bits(bits, fs, t0);  // its barriers order the writes of roff, too
+    pick_bits(bits, fs, t0);  // its barriers order the writes of off, too
 #pragma unroll
     for (int j = 0; j < kMaxRemote; ++j) {
       const int r = fs[j] - t0;
@@ -473,10 +502,17 @@ __global__ __launch_bounds__(256) void expert_fill_kernel(PackArgs a) {
       const uint64_t* b = bits + 4 * r;
       int rank = __popcll(b[w] & ((1ull << lane) - 1ull));
       for (int i = 0; i < w; ++i) rank += __popcll(b[i]);
-      const int base = at[j] + (SCAN ? roff[fs[j] * Hkv + kh] : 0);
+      const int base = at[j] + (SCAN ? (int)off[fs[j] * Hkv + kh] : 0);
       a.rows[base + rank] = ((s * Hq + h) << 3) | j;
     }
   }
+  if (a.tiles == nullptr) return;
+  const int wg = h * nblk + blk, nwg = nblk * Hq;
+  const int ntiles = SCAN ? (int)(total >> 32) : a.tile_off[E];
+  for (int e = wg; e < E; e += nwg)
+    write_tiles(a, e, SCAN ? (int)off[e] : a.row_off[e],
+                SCAN ? (int)(off[e] >> 32) : a.tile_off[e], ntiles);
+  clear_tiles(a, wg, nwg, ntiles);
 }
 
 int64_t pick_blocks(int T) { return ((int64_t)T + 255) / 256; }
@@ -595,7 +631,7 @@ extern "C" int moba_hip_pack_experts(const int* sel, int T, int Hq, int Hkv, int
   if (T < 1) return MOBA_OK;
   hipStream_t st = (hipStream_t)stream;
   const PackArgs a = {sel, T, Hq, Hkv, R, cu_chunk, chunk_batch, cu_seqlens, filtered, F,
-                      block_rows, counts, row_off, tile_off, rows, work};
+                      block_rows, counts, row_off, tile_off, rows, work, nullptr, 0};
   hipLaunchKernelGGL(pick_count_kernel, dim3((unsigned)pick_blocks(T), Hq), dim3(256), 0, st, a);
   launch_pack(a, st);
   return moba_launch_status("pack_experts");
@@ -608,8 +644,9 @@ extern "C" int moba_hip_prefill_route(const void* q, const void* k, int dtype, i
                                       const int* cu_seqlens, const int* filtered, int R, int F,
                                       int block_rows, float* means, int* sel, float* gate,
                                       int* counts, int* row_off, int* tile_off, int* rows,
-                                      int* work, void* stream) {
+                                      int* tiles, int n_tiles, int* work, void* stream) {
   if (F <= 0) return MOBA_OK;
+  if (tiles && (n_tiles < 1 || block_rows > 511 || ((uintptr_t)tiles & 15))) { moba_set_error("prefill_route: tiles must hold n_tiles 16-byte aligned entries of at most 511 rows"); return MOBA_ERR_ARG; }
   if (Hkv < 1 || Hq < 1) { moba_set_error("prefill_route: bad head counts"); return MOBA_ERR_ARG; }
   if (int rc = check_pack(T, Hq, Hkv, R, work)) return rc;
   if (int rc = moba_hip_chunk_means(k, dtype, T, Hkv, D, chunk_start, F, chunk, precision, means,
@@ -618,6 +655,6 @@ extern "C" int moba_hip_prefill_route(const void* q, const void* k, int dtype, i
   if (int rc = route_prefill(q, dtype, T, Hq, Hkv, D, means, cu_chunk, nchunk, chunk_batch,
                              first_chunk, R, F, sel, gate, work, st)) return rc;
   launch_pack({sel, T, Hq, Hkv, R, cu_chunk, chunk_batch, cu_seqlens, filtered, F, block_rows,
-               counts, row_off, tile_off, rows, work}, st);
+               counts, row_off, tile_off, rows, work, (int4*)tiles, n_tiles}, st);
   return moba_launch_status("prefill_route");
 }

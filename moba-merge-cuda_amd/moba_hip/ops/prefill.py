@@ -212,7 +212,7 @@ def get_plan(cu, chunk, hq, hkv, head_dim, topk, device, fallback=False):
 
 class RouteResult:
     """Device routing state shared by the forward and the backward."""
-    __slots__ = ("sel", "counts", "row_off", "tile_off", "rows", "means")
+    __slots__ = ("sel", "counts", "row_off", "tile_off", "rows", "tiles", "means")
 
 
 def route(plan: PrefillPlan, q, k, precision: int, want_gate=False):
@@ -230,6 +230,7 @@ def route(plan: PrefillPlan, q, k, precision: int, want_gate=False):
     r.row_off = torch.empty(E + 1, dtype=torch.int32, device=dev)
     r.tile_off = torch.empty(E + 1, dtype=torch.int32, device=dev)
     r.rows = torch.empty(max(1, T * hq * R), dtype=torch.int32, device=dev)
+    r.tiles = torch.empty((-(-plan.max_remote_tiles // 8) * 8, 4), dtype=torch.int32, device=dev)
     gate = torch.empty((F, hq, T), dtype=torch.float32, device=dev) if want_gate else None
     work = torch.empty(max(1, _lib.load().moba_hip_pack_experts_work(T, hq, plan.hkv, F)),
                        dtype=torch.int32, device=dev)
@@ -238,7 +239,8 @@ def route(plan: PrefillPlan, q, k, precision: int, want_gate=False):
               len(plan.chunk_batch), plan.ptr("chunk_batch"), plan.ptr("first_chunk"),
               plan.ptr("cu_seqlens"), plan.ptr("filtered"), R, F, plan.block_rows,
               r.means.data_ptr(), r.sel.data_ptr(), _lib.ptr(gate), r.counts.data_ptr(),
-              r.row_off.data_ptr(), r.tile_off.data_ptr(), r.rows.data_ptr(), work.data_ptr(), st)
+              r.row_off.data_ptr(), r.tile_off.data_ptr(), r.rows.data_ptr(), r.tiles.data_ptr(),
+              r.tiles.shape[0], work.data_ptr(), st)
     return (r, gate) if want_gate else r
 
 
@@ -253,12 +255,13 @@ def forward(plan: PrefillPlan, q, k, v, rt: RouteResult | None):
     if R:
         part_o = torch.empty((T * hq * R, d), dtype=q.dtype, device=dev)
         part_ml = torch.empty((T * hq * R, 2), dtype=torch.float32, device=dev)
-    _lib.call("moba_hip_prefill_fwd", q.data_ptr(), k.data_ptr(), v.data_ptr(),
+    _lib.call("moba_hip_prefill_fwd_tiles", q.data_ptr(), k.data_ptr(), v.data_ptr(),
               DTYPE_CODE[q.dtype], T, hq, plan.hkv, d, d ** -0.5,
               plan.ptr("att_chunk"), plan.ptr("self_tiles"), plan.n_self_tiles,
               _lib.ptr(rt.sel) if R else None, R, plan.ptr("filtered"), plan.num_experts,
               _lib.ptr(rt.tile_off) if R else None, _lib.ptr(rt.row_off) if R else None,
               _lib.ptr(rt.counts) if R else None, _lib.ptr(rt.rows) if R else None,
+              _lib.ptr(rt.tiles) if R else None,
               plan.max_remote_tiles if R else 0, _lib.ptr(part_o), _lib.ptr(part_ml),
               out.data_ptr(), lse.data_ptr(), _lib.stream_of(dev))
     return out, lse
@@ -284,6 +287,7 @@ def backward(plan: PrefillPlan, q, k, v, out, lse, dout, rt: RouteResult | None)
             _lib.ptr(rt.sel) if R else None, R, plan.ptr("filtered"), plan.num_experts,
             _lib.ptr(rt.tile_off) if R else None, _lib.ptr(rt.row_off) if R else None,
             _lib.ptr(rt.counts) if R else None, _lib.ptr(rt.rows) if R else None,
+            _lib.ptr(rt.tiles) if R else None,
             plan.max_remote_tiles if R else 0, delta.data_ptr(), _lib.ptr(part_dq),
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr()]
     ks = plan.kv_splits
@@ -294,11 +298,11 @@ def backward(plan: PrefillPlan, q, k, v, out, lse, dout, rt: RouteResult | None)
     pack = (torch.empty(T * hq * R * (4 * d + 8), dtype=torch.uint8, device=dev)
             if R and d <= 128 else None)
     st = _lib.stream_of(dev)
-    _lib.call("moba_hip_prefill_bwd", *args, 1, ks, _lib.ptr(part_dkv), _lib.ptr(pack), st)
+    _lib.call("moba_hip_prefill_bwd_tiles", *args, 1, ks, _lib.ptr(part_dkv), _lib.ptr(pack), st)
     events = DKDV_EVENTS
     if events is not None:
         events[0].record()
-    _lib.call("moba_hip_prefill_bwd", *args, 2, ks, _lib.ptr(part_dkv), _lib.ptr(pack), st)
+    _lib.call("moba_hip_prefill_bwd_tiles", *args, 2, ks, _lib.ptr(part_dkv), _lib.ptr(pack), st)
     if events is not None:
         events[1].record()
     return dq, dk, dv

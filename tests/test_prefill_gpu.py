@@ -437,3 +437,44 @@ def test_expert_lists(cuda_device, hq, hkv, lens, chunk, topk):
         np.testing.assert_array_equal(r.row_off.cpu().numpy(), np.r_[0, counts.cumsum()])
         np.testing.assert_array_equal(r.tile_off.cpu().numpy(), np.r_[0, tiles.cumsum()])
         np.testing.assert_array_equal(r.rows.cpu().numpy()[:counts.sum()], np.concatenate(rows))
+
+
+@pytest.mark.parametrize("hq,hkv,dim,lens,chunk", [(4, 2, 64, (700, 300), 64),
+                                                   (6, 1, 128, (1500,), 300)])
+def test_remote_tiles_given_or_searched(cuda_device, monkeypatch, hq, hkv, dim, lens, chunk):
+    """The entries that search tile_off for a workgroup's expert and those
+    that are given every workgroup's tile: the same bits, and a tile list with
+    exactly the tiles that the counts spell out."""
+    from moba_hip.ops import prefill as P
+    q, k, v, cu, ml, g = prefill_inputs(hq, hkv, dim, lens, torch.bfloat16, seed=29)
+    cfg = {"chunk_size": chunk, "topk": 3}
+    plan, rt, _ = _gpu_route(q, k, cu, cfg)
+    tiles = rt.tiles.cpu().numpy().reshape(-1, 4)
+    counts, row_off = rt.counts.cpu().numpy(), rt.row_off.cpu().numpy()
+    expect = []
+    for e, n in enumerate(counts):
+        c = plan.filtered[e // hkv]
+        for r0 in range(0, n, plan.block_rows):
+            expect.append((plan.cu_chunk[c], plan.cu_chunk[c + 1] - plan.cu_chunk[c],
+                           row_off[e] + r0,
+                           (e % hkv) << 9 | min(plan.block_rows, n - r0)))
+    per = -(-len(expect) // 8)
+    for L, got in enumerate(tiles):
+        t = (L % 8) * per + L // 8
+        ok = L // 8 < per and t < len(expect)
+        assert tuple(got) == (expect[t] if ok else (0, 0, 0, 0)), (L, t)
+
+    def grads():
+        qr, kr, vr, out, lse, _ = _run(q, k, v, cu, ml, cfg)
+        return out, lse, *torch.autograd.grad(out, (qr, kr, vr), grad_outputs=g)
+    given = grads()
+    call, at = P._lib.call, {"moba_hip_prefill_fwd_tiles": 20, "moba_hip_prefill_bwd_tiles": 25}
+
+    def searched(name, *args):
+        if name in at:
+            i = at[name]
+            args, name = args[:i] + args[i + 1:], name[:-len("_tiles")]
+        call(name, *args)
+    monkeypatch.setattr(P._lib, "call", searched)
+    for a, b in zip(given, grads()):
+        assert torch.equal(a, b)
