@@ -381,62 +381,44 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
     if constexpr (REMOTE) {
       uint16_t* po = a.part_dq + (int64_t)slot[qb] * D;
 #pragma unroll
-      for (int db = 0; db < NDB; ++db)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int d0 = db * 32 + 8 * j + 4 * hh;
-          if (d0 < D) {
-            f32x4_t o;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = acc[qb][db][4 * j + i] * a.scale;
-            u16x4_t ob;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) ob[i] = from_f32<DT>(o[i]);
-            *reinterpret_cast<u16x4_t*>(po + d0) = ob;
-          }
-        }
+      for (int db = 0; db < NDB; ++db) store_block<DT>(po, acc[qb][db], a.scale, db, 8 * hh, D);
     } else {
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[qb][db][r] *= a.scale;
-      // one slot per iteration, all of its loads issued together: slots
-      // below R are in the row's allocation, columns past D are clamped and
-      // masked, unselected slots (sel < 0) add zero
+      // one slot per iteration, its loads issued together: slots below R are
+      // in the row's allocation, columns past D are clamped (they reach only
+      // entries that are not stored), unselected slots (sel < 0) add zero
       for (int jj = 0; jj < a.R; ++jj) {
         const int64_t sl = row * a.R + jj;
         const bool on = a.sel[sl] >= 0;
         const uint16_t* po = a.part_dq + sl * D;
-        u16x4_t o[NDB][4];
+        constexpr int NBL = NDB <= 4 ? NDB : 2;
 #pragma unroll
-        for (int db = 0; db < NDB; ++db)
+        for (int d4 = 0; d4 < NDB; d4 += NBL) {
+          u16x8_t o[NBL][2];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int d0 = db * 32 + 8 * j + 4 * hh;
-            o[db][j] = *reinterpret_cast<const u16x4_t*>(po + (d0 < D ? d0 : 0));
-          }
+          for (int db = 0; db < NBL; ++db)
 #pragma unroll
-        for (int db = 0; db < NDB; ++db)
+            for (int m = 0; m < 2; ++m) {
+              const int d = (d4 + db) * 32 + 16 * m + 8 * hh;
+              o[db][m] = ld8(po + (d < D ? d : 0));
+            }
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const bool ok = on && db * 32 + 8 * j + 4 * hh < D;
+          for (int db = 0; db < NBL; ++db)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[qb][db][4 * j + i] += ok ? to_f32<DT>(o[db][j][i]) : 0.0f;
-          }
+            for (int m = 0; m < 2; ++m) {
+              float x[8];
+              spread_piece<DT>(o[db][m], x);
+#pragma unroll
+              for (int i = 0; i < 8; ++i) acc[qb][d4 + db][8 * m + i] += on ? x[i] : 0.0f;
+            }
+        }
       }
       uint16_t* orow = a.dq + row * D;
 #pragma unroll
-      for (int db = 0; db < NDB; ++db)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int d0 = db * 32 + 8 * j + 4 * hh;
-          if (d0 < D) {
-            u16x4_t o;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = from_f32<DT>(acc[qb][db][4 * j + i]);
-            *reinterpret_cast<u16x4_t*>(orow + d0) = o;
-          }
-        }
+      for (int db = 0; db < NDB; ++db) store_block<DT>(orow, acc[qb][db], 1.0f, db, 8 * hh, D);
     }
   }
 }

@@ -18,15 +18,18 @@
 //    ascending-slot order (global softmax: m = max l, O = sum e^{l-m} o / z,
 //    L = m + log z) and writes the final O (input dtype) and LSE (fp32).
 //
-// Tile math (per wave: 2 blocks of 32 query rows, key tiles of 64):
+// Tile math (per wave: QB blocks of 32 query rows, key tiles of fwd_keys):
 //   S^T = K Q^T      (A = K rows from LDS, B = Q fragment in registers)
 //   O^T += V^T P^T   (A = V^T read from the row-major V tile with the gfx950
 //                     transposed LDS read, B = P straight from the S^T
 //                     accumulators: the D-layout of S^T is the B-layout of P^T
 //                     up to a fixed key order, which the transposed read follows)
-// Each K / V^T fragment read from LDS feeds the MFMAs of both query blocks, and
-// the next K/V tile is prefetched into registers while the current one computes.
 // so every per-query quantity (running max, sum, rescale) is lane-uniform.
+// One body serves masked and full tiles, the mask behind a uniform branch
+// (two bodies held the accumulators in different registers).  Rows are written
+// and partials read in 16-byte pieces (store_block): in the 8-byte pieces of
+// the accumulator layout the self kernel took 1346 instead of 1190 us at T
+// 32768, 32 heads, chunk 4096, and 170 instead of 147 at 8 heads, chunk 512.
 #include <type_traits>
 
 #include "common.h"
@@ -60,12 +63,23 @@ struct FwdArgs {
   float* lse;
 };
 
-constexpr int kBN = 64;   // keys per LDS tile
+// Keys per LDS tile, and the waves per SIMD the registers are held to.  What
+// hides the latencies of a tile (LDS operands, exponentials, the barrier) is
+// another workgroup on the CU, so the tile is cut until one more fits: 32 keys
+// give three waves per SIMD at 128 dims (139 registers; 64 keys: two) and two
+// at 256 (242 registers, 64 KB of LDS; 64 keys: one wave, 128 KB).  Remote /
+// self forward, us, 64 -> 32 keys: T 32768, 32 heads, D 128, chunk 4096
+// 3570 / 1425 -> 3415 / 1346; T 8192, 16/4 heads, D 256, chunk 1024 455 / 206
+// -> 289 / 171.  A fourth wave at 128 dims spills and is slower (3510 / 1460),
+// and so are 32 keys up to 64 dims (16/2 heads, T 16384: remote 264 -> 279).
+template <int DP> constexpr int fwd_keys() { return DP <= 64 ? 64 : 32; }
+template <int DP> constexpr int fwd_waves() { return DP > 64 && DP <= 128 ? 3 : 2; }
 constexpr float kRescaleSlack = 8.0f;  // log2 headroom before O is rescaled
 
 template <int DT, int DP, bool REMOTE, int QB>
-__global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs a) {
+__global__ __launch_bounds__(256, fwd_waves<DP>()) void fwd_kernel(FwdArgs a) {
   constexpr int NKS = DP / 16;  // k-steps of the QK^T contraction
+  constexpr int kBN = fwd_keys<DP>(), NKB = kBN / 32;  // keys per tile, 32-key blocks
   constexpr int NDB = DP / 32;  // 32-row d blocks of O^T
   constexpr int TILE = kBN * DP;           // elements of one K or V tile
   constexpr int NB = DP / 8;                // 16-byte blocks per tile row
@@ -210,14 +224,13 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
   const uint32_t trb0 = swz_tr_base<DP>(lane, 0), trb1 = swz_tr_base<DP>(lane, 1);
 
   const int ntiles = (n_keys + kBN - 1) / kBN;
-  auto tile = [&](const uint16_t* Kb, const uint16_t* Vb, const int it, auto mask_tag) {
-    constexpr bool MASK = decltype(mask_tag)::value;
+  auto tile = [&](const uint16_t* Kb, const uint16_t* Vb, const int it, const bool mask) {
     const int kt0 = k_lo + it * kBN;
     const uint32_t kq = opaque(kbase0), t0 = opaque(trb0), t1 = opaque(trb1);
-    f32x16_t sacc[QB][2];
+    f32x16_t sacc[QB][NKB];
     wave_prio<1>();
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
+    for (int kb = 0; kb < NKB; ++kb) {
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) sacc[qb][kb] = zero16();
 #pragma unroll
@@ -228,11 +241,11 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
       }
     }
     wave_prio<0>();
-    if constexpr (MASK) {
+    if (mask) {  // uniform
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int key = kt0 + kb * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
@@ -240,12 +253,12 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
             sacc[qb][kb][r] = ok ? sacc[qb][kb][r] : -INFINITY;
           }
     }
-    u16x8_t pv[QB][2][2];
+    u16x8_t pv[QB][NKB][2];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       float mx = -INFINITY;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sacc[qb][kb][r]);
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c2;
@@ -267,7 +280,7 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
       const float nm = -m_run[qb];
       float ps = 0.0f;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
+      for (int kb = 0; kb < NKB; ++kb) {
         float p[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -283,7 +296,7 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const uint32_t ro = (kb * 32 + t * 16) * DP * 2;
@@ -305,7 +318,7 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
     // (the wave still joins the stage barriers)
     if (!REMOTE && kt0 > s_wave0 + 32 * QB - 1) return;
     const bool need_mask = (kt0 + kBN > k_hi) || (!REMOTE && kt0 + kBN - 1 > s_wave0);
-    if (need_mask) tile(Kb, Vb, it, std::true_type{}); else tile(Kb, Vb, it, std::false_type{});
+    tile(Kb, Vb, it, need_mask);
   };
   stage_sync();
   for (int it = 0; it < ntiles; it += 2) {
@@ -327,20 +340,7 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
       const float inv = 1.0f / l;
       uint16_t* po = a.part_o + (int64_t)slot[qb] * D;
 #pragma unroll
-      for (int db = 0; db < NDB; ++db)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int d0 = db * 32 + 8 * j + 4 * hh;
-          if (d0 < D) {
-            f32x4_t o;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = oacc[qb][db][4 * j + i] * inv;
-            u16x4_t ob;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) ob[i] = from_f32<DT>(o[i]);
-            *reinterpret_cast<u16x4_t*>(po + d0) = ob;
-          }
-        }
+      for (int db = 0; db < NDB; ++db) store_block<DT>(po, oacc[qb][db], inv, db, 8 * hh, D);
       // partial stored as (running max, sum) in the log2 domain: merging
       // them is exact in fp32 even when |logits| is huge (an LSE would round
       // log2(l) away next to a large max)
@@ -371,40 +371,38 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void fwd_kernel(FwdArgs 
         const int sv = a.sel[sl];
         const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + 2 * sl);
         const uint16_t* po = a.part_o + sl * D;
-        u16x4_t o[NDB][4];
-#pragma unroll
-        for (int db = 0; db < NDB; ++db)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int d0 = db * 32 + 8 * j + 4 * hh;
-            o[db][j] = *reinterpret_cast<const u16x4_t*>(po + (d0 < D ? d0 : 0));
-          }
         // an unselected slot's data may be stale or NaN: select, never 0 * x
         const float w = sv >= 0 ? ml.y * fast_exp2(ml.x - M2) : 0.0f;
         z += w;
+        // up to four d blocks in flight (two where the accumulators leave no
+        // room for more)
+        constexpr int NBL = NDB <= 4 ? NDB : 2;
 #pragma unroll
-        for (int db = 0; db < NDB; ++db)
+        for (int d4 = 0; d4 < NDB; d4 += NBL) {
+          u16x8_t o[NBL][2];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const bool ok = sv >= 0 && db * 32 + 8 * j + 4 * hh < D;
+          for (int db = 0; db < NBL; ++db)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) oacc[qb][db][4 * j + i] += ok ? w * to_f32<DT>(o[db][j][i]) : 0.0f;
-          }
+            for (int m = 0; m < 2; ++m) {
+              const int d = (d4 + db) * 32 + 16 * m + 8 * hh;
+              o[db][m] = ld8(po + (d < D ? d : 0));
+            }
+#pragma unroll
+          for (int db = 0; db < NBL; ++db)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+              float x[8];
+              spread_piece<DT>(o[db][m], x);
+#pragma unroll
+              for (int i = 0; i < 8; ++i)
+                oacc[qb][d4 + db][8 * m + i] += sv >= 0 ? w * x[i] : 0.0f;
+            }
+        }
       }
       const float invz = 1.0f / z;
       uint16_t* orow = a.out + row * D;
 #pragma unroll
-      for (int db = 0; db < NDB; ++db)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int d0 = db * 32 + 8 * j + 4 * hh;
-          if (d0 < D) {
-            u16x4_t o;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = from_f32<DT>(oacc[qb][db][4 * j + i] * invz);
-            *reinterpret_cast<u16x4_t*>(orow + d0) = o;
-          }
-        }
+      for (int db = 0; db < NDB; ++db) store_block<DT>(orow, oacc[qb][db], invz, db, 8 * hh, D);
       if (hh == 0) a.lse[row] = (M2 + log2f(z)) * kLn2;
     }
   }

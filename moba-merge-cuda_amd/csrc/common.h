@@ -277,6 +277,46 @@ MOBA_DEV void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Rows of a transposed accumulator (D layout: lane l holds column l % 32,
+// entries 8j + 4(l/32) + i of each 32-entry block) as 16-byte pieces: lanes l
+// and l + 32 exchange halves (v_permlane32_swap), after which lane l holds
+// entries 16m .. 16m + 7 of its column and lane l + 32 entries 16m + 8 ..
+// 16m + 15.  Half the memory instructions of the 8-byte pieces that the
+// layout has in place.  The swap is its own inverse.
+MOBA_DEV void swap_halves(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+// Column `row` of block db, scaled, in the 16-bit type.  d0 = 8 * (lane / 32).
+template <int DT>
+MOBA_DEV void store_block(uint16_t* row, const f32x16_t& v, float scale, int db, int d0, int D) {
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = v[8 * m + i] * scale;
+    uint32_t a0 = pack2<DT>(x[0], x[1]), a1 = pack2<DT>(x[2], x[3]);
+    uint32_t b0 = pack2<DT>(x[4], x[5]), b1 = pack2<DT>(x[6], x[7]);
+    swap_halves(a0, b0);
+    swap_halves(a1, b1);
+    const int d = db * 32 + 16 * m + d0;
+    if (d < D) st8(row + d, __builtin_bit_cast(u16x8_t, (u32x4_t){a0, a1, b0, b1}));
+  }
+}
+// The reverse of store_block on a piece loaded from d = 32 db + 16 m + d0:
+// the 8 values of accumulator entries 8m .. 8m + 7.
+template <int DT> MOBA_DEV void spread_piece(const u16x8_t& piece, float (&x)[8]) {
+  u32x4_t w = __builtin_bit_cast(u32x4_t, piece);
+  uint32_t a0 = w[0], a1 = w[1], b0 = w[2], b1 = w[3];
+  swap_halves(a0, b0);
+  swap_halves(a1, b1);
+  unpack2<DT>(a0, x[0], x[1]);
+  unpack2<DT>(a1, x[2], x[3]);
+  unpack2<DT>(b0, x[4], x[5]);
+  unpack2<DT>(b1, x[6], x[7]);
+}
+
 // 32-row query blocks per wave in the query-major attention kernels (forward
 // and dQ); a workgroup of 4 waves covers 128 * attn_qb rows.  One block per
 // wave leaves room for two waves per SIMD.

@@ -123,6 +123,16 @@ def test_forward_backward_vs_fp64(cuda_device, hq, hkv, dim, lens, chunk, topk, 
         assert_grad_close(a, e, dtype, name, mean_tol=dv_mean if name == "dv" else None)
 
 
+@pytest.mark.parametrize("dim", [24, 72, 120, 136, 248, 256])
+@pytest.mark.parametrize("chunk", [31, 33, 65])
+def test_head_dim_and_key_tile_edges(cuda_device, dim, chunk):
+    """Chunks that end one key before, after and well past a 32- or 64-key
+    tile, with head dims whose last 16-column pair is half there (rows are
+    written and read in 16-byte pieces, two lanes to a pair) in every width."""
+    test_forward_backward_vs_fp64(cuda_device, 4, 2, dim, (3 * chunk + 5, 40), chunk, 3,
+                                  torch.bfloat16)
+
+
 def test_repeat_bitwise(cuda_device):
     q, k, v, cu, ml, g = prefill_inputs(8, 2, 64, (257, 129), torch.bfloat16, seed=362)
     cfg = {"chunk_size": 16, "topk": 4}
