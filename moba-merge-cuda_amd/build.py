@@ -39,18 +39,10 @@ def _headers():
     return max((h.stat().st_mtime for h in hs), default=0.0)
 
 
-# Per-source flag changes.  attn_dkdv.hip runs one wave per SIMD: its dK / dV
-# accumulators belong in AGPRs, so it is built without the VGPR-form flag.
-NO_VGPR_FORM = {"attn_dkdv.hip"}
-
-
 def _flags(src: Path):
     if src.suffix == ".cpp":  # host-only sources: the host compiler, HIP runtime API only
         return ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result", "-D__HIP_PLATFORM_AMD__",
                 "-I/opt/rocm/include"]
-    if src.name in NO_VGPR_FORM:
-        i = FLAGS.index("-amdgpu-mfma-vgpr-form")
-        return FLAGS[:i - 1] + FLAGS[i + 1:]
     return FLAGS
 
 

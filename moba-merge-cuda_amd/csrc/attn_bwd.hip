@@ -925,8 +925,7 @@ int launch_bwd(const BwdArgs& a, int n_self, int n_kv, int max_remote, int parts
     // kKvTileKeys keys per workgroup in every kernel; the host's key tiles match
     const int n_wg = n_kv * a.kv_splits;
     if (a.kv_splits > 1) {
-      constexpr int rows = 32 * dkdv_qb<DP>();  // query rows per tile of every key-major kernel
-      hipLaunchKernelGGL(dkdv_sched_kernel<DP <= 128 ? 64 : rows>, dim3(1), dim3(1024), 0, st, a,
+      hipLaunchKernelGGL(dkdv_sched_kernel<kv_rows<DP>()>, dim3(1), dim3(1024), 0, st, a,
                          n_kv, n_wg, const_cast<int*>(a.kv_sched), const_cast<int*>(a.kv_seg));
     }
     if constexpr (DP <= 128) {

@@ -22,6 +22,15 @@
 // P and dS never leave registers and the waves never wait for each other
 // inside a tile: one barrier per tile, where the LDS stages rotate.  Used for
 // head dims <= 64, where the registers allow two waves per SIMD.
+//
+// At 64 dims a tile's element-wise work (an exponential, two products and two
+// conversions per score) takes about as long as its 32 MFMAs, so the two are
+// laid side by side in the wave's own stream: the first 32 rows' exponentials
+// between the second 32 rows' S / dP products, the second's between the
+// first's dV / dK products, with LDS operands read two steps ahead and the
+// mask behind a uniform branch (a second, masked body took 251 registers).  T 16384, 14/2 heads, chunk 2048: 735 -> 655 us; the ragged
+// fp16 batch of 12238 tokens, 28/4 heads: 331 -> 285 us (one body alone 690 /
+// 302; three or four steps ahead the same; tiles of 32 rows 750 / 330).
 #include <type_traits>
 
 #include "common.h"
@@ -31,7 +40,6 @@ namespace moba {
 namespace {
 
 constexpr int kWaveKeys = 32;   // keys per wave
-constexpr int kRows = 64;       // query rows per tile
 constexpr int kStages = 3;      // LDS stages of (Q, dO) tiles
 
 // s_waitcnt vmcnt(N), other counters untouched (N < 16).
@@ -41,7 +49,8 @@ template <int N> MOBA_DEV void wait_vmcnt() {
 }
 
 template <int DT, int DP>
-__global__ __launch_bounds__(256, 1) void dkdv1_kernel(BwdArgs a) {
+__global__ __launch_bounds__(256, 2) void dkdv1_kernel(BwdArgs a) {
+  constexpr int kRows = kv_rows<DP>();
   constexpr int NKS = DP / 16, NDB = DP / 32, QB = kRows / 32;
   constexpr int NB = DP / 8;                    // 16-byte blocks per row
   constexpr int NDMA = kRows * NB / 256;        // blocks per thread per operand
@@ -140,12 +149,12 @@ __global__ __launch_bounds__(256, 1) void dkdv1_kernel(BwdArgs a) {
       dma_lds16(make_rsrc(srcq, nb), Qd + jb * 8, off, 0);
       dma_lds16(make_rsrc(srcg, nb), Gd + jb * 8, off, 0);
     }
-    if (lane < 16) {  // wave w: lse_k and delta of rows 16w .. 16w + 15
-      const int q = wave_s * 16 + lane;
+    if (lane < kRows / 4) {  // wave w: lse_k and delta of a quarter of the rows
+      const int q = wave_s * (kRows / 4) + lane;
       const uint32_t lb = is_self ? lbytes : plbytes;
       const uint32_t off = q < nvalid ? (uint32_t)(r0 + q * rstride) * 4 : lb;
-      dma_lds4(make_rsrc(is_self ? a.lse_k : a.pack_lse_k, lb), Ld + wave_s * 16, off, 0);
-      dma_lds4(make_rsrc(is_self ? a.delta : a.pack_delta, lb), Ld + kRows + wave_s * 16, off, 0);
+      dma_lds4(make_rsrc(is_self ? a.lse_k : a.pack_lse_k, lb), Ld + wave_s * (kRows / 4), off, 0);
+      dma_lds4(make_rsrc(is_self ? a.delta : a.pack_delta, lb), Ld + kRows + wave_s * (kRows / 4), off, 0);
     }
   };
   const uint32_t kq0 = swz_b128_base<DP>(lane);
@@ -171,8 +180,7 @@ __global__ __launch_bounds__(256, 1) void dkdv1_kernel(BwdArgs a) {
   for (int i = 0; i < NDB; ++i) { dk[i] = zero16(); dv[i] = zero16(); }
 
   auto compute = [&](const uint16_t* Qb, const uint16_t* Gb, const float* Lb, const int it,
-                     auto mask_tag) __attribute__((always_inline)) {
-    constexpr bool MASK = decltype(mask_tag)::value;
+                     const bool mask) __attribute__((always_inline)) {
     const uint32_t kq = opaque(kq0), t0 = opaque(trb0), t1 = opaque(trb1);
     const bool is_self = it < G * n_self;
     const int sq0 = is_self ? self_begin + (it % n_self) * kRows : 0;
@@ -188,40 +196,71 @@ __global__ __launch_bounds__(256, 1) void dkdv1_kernel(BwdArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) { sp[qb][4 * j + i] = l4[i]; dp[qb][4 * j + i] = d4[i]; }
       }
+    constexpr int NA = QB * NKS, NB2 = QB * 2 * NDB, PF = 2;
+    u16x8_t ring[PF][2];
+    auto rda = [&](int i) __attribute__((always_inline)) {  // block i / NKS, k-step i % NKS
+      const uint32_t o = (i / NKS) * 32 * DP * 2 + swz_b128<DP>(kq, i % NKS);
+      ring[i % PF][0] = lds8(Qb, o);
+      ring[i % PF][1] = lds8(Gb, o);
+    };
+    auto rdb = [&](int j) __attribute__((always_inline)) {  // 16-row group j / NDB, d block j % NDB
+      const uint32_t ro = (j / NDB) * 16 * DP * 2;
+      const uint32_t x0 = ro + swz_tr<DP>(t0, j % NDB), x1 = ro + swz_tr<DP>(t1, j % NDB);
+      ring[(NA + j) % PF][0] = lds_tr8(Gb, x0, x1);
+      ring[(NA + j) % PF][1] = lds_tr8(Qb, x0, x1);
+    };
+    // operands of step n of the whole sequence (NA steps, then NB2), read PF
+    // steps ahead
+    auto rd = [&](int n) __attribute__((always_inline)) {
+      if (n < NA) rda(n); else if (n < NA + NB2) rdb(n - NA);
+    };
+    // a masked pair's P becomes exp2(-inf) = 0, whatever its product was
+    auto cut = [&](int qb) __attribute__((always_inline)) {
 #pragma unroll
-    for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        const uint32_t o = qb * 32 * DP * 2 + swz_b128<DP>(kq, ks);
-        sp[qb] = mfma32<DT>(lds8(Qb, o), kf[ks], sp[qb]);
-        dp[qb] = mfma32<DT>(lds8(Gb, o), vf[ks], dp[qb]);
+      for (int r = 0; r < 16; ++r) {
+        const int row = sq0 + qb * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
+        sp[qb][r] = (mykey < c_hi && (!is_self || mykey <= row)) ? sp[qb][r] : INFINITY;
       }
+    };
     // P and -dS as A operands: P = exp2(c2 (S - lse_k)), -dS = P (delta - dP)
     u16x8_t pa[QB][2], da[QB][2];
+    auto soft = [&](int qb, int r0, int n) __attribute__((always_inline)) {
 #pragma unroll
-    for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r0 = qb * 32 + 8 * j + 4 * hh;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float p = fast_exp2(sp[qb][4 * j + i] * nc2);
-          if constexpr (MASK) p = (mykey < c_hi && (!is_self || mykey <= sq0 + r0 + i)) ? p : 0.0f;
-          pa[qb][j >> 1][(j & 1) * 4 + i] = from_f32<DT>(p);
-          da[qb][j >> 1][(j & 1) * 4 + i] = from_f32<DT>(p * dp[qb][4 * j + i]);
-        }
+      for (int r = r0; r < r0 + n; ++r) {
+        const float p = fast_exp2(sp[qb][r] * nc2);
+        pa[qb][r >> 3][r & 7] = from_f32<DT>(p);
+        da[qb][r >> 3][r & 7] = from_f32<DT>(p * dp[qb][r]);
       }
+    };
 #pragma unroll
-    for (int i = 0; i < NDB; ++i)
+    for (int n = 0; n < PF; ++n) rd(n);
 #pragma unroll
-      for (int qb = 0; qb < QB; ++qb)
+    for (int n = 0; n < NA; ++n) {
+      const int qb = n / NKS, ks = n % NKS;
+      const u16x8_t xq = ring[n % PF][0], xg = ring[n % PF][1];
+      rd(n + PF);
+      sp[qb] = mfma32<DT>(xq, kf[ks], sp[qb]);
+      dp[qb] = mfma32<DT>(xg, vf[ks], dp[qb]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (ks == NKS - 1 && mask) cut(qb);  // uniform
+      if (qb > 0) {
+        soft(qb - 1, ks * (16 / NKS), 16 / NKS);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const uint32_t ro = (qb * 32 + t * 16) * DP * 2;
-          const uint32_t x0 = ro + swz_tr<DP>(t0, i), x1 = ro + swz_tr<DP>(t1, i);
-          dv[i] = mfma32<DT>(pa[qb][t], lds_tr8(Gb, x0, x1), dv[i]);
-          dk[i] = mfma32<DT>(da[qb][t], lds_tr8(Qb, x0, x1), dk[i]);
-        }
+    for (int n = 0; n < NB2; ++n) {
+      const int m = NA + n, qb = n / (2 * NDB), t = (n / NDB) % 2, i = n % NDB;
+      const u16x8_t xg = ring[m % PF][0], xq = ring[m % PF][1];
+      rd(m + PF);
+      dv[i] = mfma32<DT>(pa[qb][t], xg, dv[i]);
+      dk[i] = mfma32<DT>(da[qb][t], xq, dk[i]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (qb == 0) {  // the last block's exponentials under the first block's products
+        soft(QB - 1, n * (16 / (2 * NDB)), 16 / (2 * NDB));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
   };
   auto run = [&](const uint16_t* Qb, const uint16_t* Gb, const float* Lb, const int it) __attribute__((always_inline)) {
     const bool is_self = it < G * n_self;
@@ -229,8 +268,7 @@ __global__ __launch_bounds__(256, 1) void dkdv1_kernel(BwdArgs a) {
     // causal rows that end before the wave's first key contribute nothing
     if (is_self && sq0 + kRows - 1 < wkey0) return;
     const bool need_mask = (wkey0 + kWaveKeys > c_hi) || (is_self && sq0 < wkey0 + kWaveKeys - 1);
-    if (need_mask) compute(Qb, Gb, Lb, it, std::true_type{});
-    else compute(Qb, Gb, Lb, it, std::false_type{});
+    compute(Qb, Gb, Lb, it, need_mask);
   };
   // Stage k of tile it is (it - it_lo) % 3.  Loads run two tiles ahead; after
   // computing tile it, each wave waits until its loads of tile it + 1 landed

@@ -42,7 +42,7 @@ namespace moba {
 namespace {
 
 constexpr int kPairKeys = 32;   // keys per wave pair
-constexpr int kRows = 64;       // query rows per tile
+constexpr int kRows = kv_rows<128>();  // query rows per tile
 // role P issues load piece k of the next tile after MFMA step kDmaAt + 2k
 // of its block (the loads then overlap the block instead of stalling the
 // start of the step)

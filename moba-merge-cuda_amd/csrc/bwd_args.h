@@ -68,6 +68,10 @@ template <int DT, int DP> void launch_dkdv2(const BwdArgs& a, int n_wg, hipStrea
 constexpr int kKvTileKeys = 128;
 __host__ __device__ inline int64_t kv_slot_floats(int D) { return (int64_t)2 * kKvTileKeys * D; }
 
+// Query rows per tile of the key-major kernel of a head-dim width: the unit of
+// the row-split schedule.
+template <int DP> constexpr int kv_rows() { return DP <= 128 ? 64 : 32; }
+
 // Work of one dK/dV workgroup: its kv tile entry and row-tile range, and the
 // partial slot it writes (-1: dK / dV directly).  Returns false for an idle
 // workgroup.  Unscheduled launches take tile blockIdx.x and all its rows.
