@@ -12,7 +12,7 @@
 //        P = exp(S*scale - LSE), dS = P (dP - Delta), dQ^T += K^T dS^T.
 //        REMOTE tiles (expert rows) write dq partials into the row's slot;
 //        SELF tiles (causal within the chunk) add the slots in ascending order.
-//   dkdv_kernel : key-major.  One workgroup owns a tile of one chunk's keys for
+//   dK / dV (attn_dkdv*.hip): key-major.  One workgroup owns a tile of one chunk's keys for
 //        one KV head and walks every query row that attends them: the causal
 //        rows of the chunk for all G heads of the group, then the expert rows
 //        that selected the chunk.  dK, dV accumulate in registers and are
@@ -423,323 +423,6 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
   }
 }
 
-// ------------------------------------------------------------------- dkdv
-// Key-major dK/dV.  A workgroup of 8 waves owns 128 keys of one chunk and one
-// KV head, as 4 pairs of waves; each pair owns 32 keys.  Within a pair the
-// work is split by role so that each wave holds only half the operands:
-//   role P (waves 0-3): K in registers; S = Q K^T, P = exp2(S*c - lse), P to
-//                       LDS (fp32), then dV += P^T dO
-//   role D (waves 4-7): V in registers; dP = dO V^T, reads P, dS = P (dP - delta),
-//                       then dK += dS^T Q
-// Query tiles of 32*QB rows (Q and dO, row-major) are double-buffered in LDS,
-// the next tile prefetched through registers and its row indices one tile
-// further ahead (a gathered expert row costs two dependent global loads: its
-// index, then its data).  The MFMA D-layout of S / dP (one key per lane) is
-// exactly the A layout of P^T / dS^T; dO and Q enter as B through the
-// transposed LDS read.  Waves w and w+4 share a SIMD, so one wave's
-// exponentials overlap its partner's MFMAs.
-constexpr int kDkdvPairKeys = 32;
-
-template <int DP> constexpr int dkdv_qb() { return DP <= 128 ? 2 : 1; }
-
-template <int DT, int DP>
-__global__ __launch_bounds__(512, 1) void dkdv_kernel(BwdArgs a) {
-  constexpr int QB = dkdv_qb<DP>();
-  constexpr int NKS = DP / 16, NDB = DP / 32;
-  constexpr int BQ = 32 * QB;                 // query rows per tile
-  constexpr int NB = DP / 8;                  // 16-byte blocks per row
-  constexpr int NDMA = (BQ * NB + 511) / 512; // blocks per thread per operand
-  constexpr int WKEYS = kDkdvPairKeys;        // keys per wave pair
-  // Q / dO tiles in two named stages (swz<DP> layout), filled by buffer loads
-  // straight into LDS while the other stage is being used.
-  __shared__ __attribute__((aligned(16))) uint16_t Q0[BQ * DP];
-  __shared__ __attribute__((aligned(16))) uint16_t G0[BQ * DP];
-  __shared__ __attribute__((aligned(16))) uint16_t Q1[BQ * DP];
-  __shared__ __attribute__((aligned(16))) uint16_t G1[BQ * DP];
-  __shared__ __attribute__((aligned(16))) float lse2s[2][BQ];
-  __shared__ __attribute__((aligned(16))) float dels[2][BQ];
-  // P handed from role P to role D as a pair of input-dtype values: Px holds
-  // P rounded to the input dtype (the operand dV uses), Pr the rounding
-  // residual, so dS = (Px + Pr)(dP - delta) sees P to about 16 mantissa bits
-  // (dS from the rounded P alone doubled the dK error at D = 256).
-  // [pair][qb][half][lane], 8 values per lane
-  __shared__ __attribute__((aligned(16))) u16x8_t Px[4][QB][2][64];
-  __shared__ __attribute__((aligned(16))) u16x8_t Pr[4][QB][2][64];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int qi = lane & 31, hh = lane >> 5;
-  const int pair = wave & 3;
-  const bool role_p = wave < 4;
-  const int wave_s = __builtin_amdgcn_readfirstlane(wave);
-  const int D = a.D, G = a.G;
-  int ti, s_lo, s_hi, slot;
-  if (!kv_work(a, ti, s_lo, s_hi, slot)) return;
-  const int* tile = a.kv_tiles + 4 * ti;
-  const int c = tile[0], kt0 = tile[1], f = tile[2], kh = tile[3];
-  if (c < 0) return;                        // padding entry of the XCD-ordered list
-  const int c_lo = a.cu_chunk[c], c_hi = a.cu_chunk[c + 1];
-  const int key0 = c_lo + kt0;              // first key of the workgroup
-  const int wkey0 = key0 + pair * WKEYS;    // first key of this pair
-  const int mykey = wkey0 + qi;             // this lane's key (B operand column)
-
-  // Uninitialised LDS could hold NaN patterns that a zero probability would
-  // not cancel; column blocks past D are never loaded and must read zero.
-#pragma unroll
-  for (int n = 0; n < NDMA; ++n) {
-    const int j = n * 512 + tid;
-    if (j < BQ * NB) {
-      st8(Q0 + j * 8, zero8()); st8(G0 + j * 8, zero8());
-      st8(Q1 + j * 8, zero8()); st8(G1 + j * 8, zero8());
-    }
-  }
-  __syncthreads();
-
-  // The two roles run as separate instantiations of the body, so each wave's
-  // code holds only its own role's registers.
-  auto body = [&](auto role_tag) {
-    constexpr bool ROLE_P = decltype(role_tag)::value;
-    // role P holds K, role D holds V (B operands: column = key, k = d)
-    u16x8_t kv[NKS];
-    const uint16_t* kvsrc = ROLE_P ? a.k : a.v;
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      const int d = ks * 16 + hh * 8;
-      const bool ok = mykey < c_hi && d < D;
-      kv[ks] = ok ? ld8(kvsrc + ((int64_t)mykey * a.Hkv + kh) * D + d) : zero8();
-    }
-    f32x16_t acc[NDB];                        // dV (role P) or dK (role D)
-#pragma unroll
-    for (int i = 0; i < NDB; ++i) acc[i] = zero16();
-
-    // query tiles: G * n_self causal tiles (rows from key0 to the chunk end, for
-    // every head of the group), then the expert's gathered rows
-    const int self_begin = key0;
-    const int n_self = (max(0, c_hi - self_begin) + BQ - 1) / BQ;
-    const int e = (f >= 0 && a.R > 0) ? f * a.Hkv + kh : -1;
-    const int n_rem = e >= 0 ? a.counts[e] : 0;
-    const int rbase = e >= 0 ? a.row_off[e] : 0;
-    const int n_tiles = G * n_self + (n_rem + BQ - 1) / BQ;
-    const int it_lo = s_lo, it_hi = min(s_hi, n_tiles);  // this workgroup's share
-
-    auto row_of = [&](int it, int qr) -> int {  // row index s*Hq+h, or -1
-      if (it < G * n_self) {
-        const int g = it / n_self, s = self_begin + (it % n_self) * BQ + qr;
-        return s < c_hi ? s * a.Hq + kh * G + g : -1;
-      }
-      const int local = (it - G * n_self) * BQ + qr;
-      return local < n_rem ? a.rows[rbase + local] >> 3 : -1;
-    };
-
-    // Thread t loads blocks j = n * 512 + t of a tile: row j / NB, physical
-    // block j % NB, logical column block (j % NB) ^ f(row).
-    int nrow[NDMA], nlrow = -1;
-    auto fetch_rows = [&](int it) {
-#pragma unroll
-      for (int n = 0; n < NDMA; ++n) {
-        const int q = (n * 512 + tid) / NB;
-        nrow[n] = q < BQ ? row_of(it, q) : -1;
-      }
-      nlrow = tid < BQ ? row_of(it, tid) : -1;
-    };
-    const uint32_t qbytes = (uint32_t)((int64_t)a.T * a.Hq * D * 2);
-    auto dma = [&](uint16_t* Qd, uint16_t* Gd) {
-#pragma unroll
-      for (int n = 0; n < NDMA; ++n) {
-        const int j = n * 512 + tid, q = j / NB;
-        const int col = swz<DP>(q, (j % NB) * 8) - q * DP;
-        if (j < BQ * NB && col < D) {
-          // rows of -1 read past the end of the tensor: zeros
-          const uint32_t off = nrow[n] >= 0 ? (uint32_t)(((int64_t)nrow[n] * D + col) * 2) : qbytes;
-          const int jb = n * 512 + wave_s * 64;  // first block of this wave's 64
-          load_lds16(make_rsrc(a.q, qbytes), Qd + jb * 8, off, 0);
-          load_lds16(make_rsrc(a.dout, qbytes), Gd + jb * 8, off, 0);
-        }
-      }
-    };
-    float lse_r = INFINITY, del_r = 0.0f;
-    auto load_ld = [&]() {
-      lse_r = nlrow >= 0 ? a.lse[nlrow] * kLog2e : INFINITY;
-      del_r = nlrow >= 0 ? a.delta[nlrow] : 0.0f;
-    };
-    auto store_ld = [&](int buf) {
-      if (tid < BQ) { lse2s[buf][tid] = lse_r; dels[buf][tid] = del_r; }
-    };
-
-    const uint32_t kq0 = swz_b128_base<DP>(lane);
-    const uint32_t trb0 = swz_tr_base<DP>(lane, 0), trb1 = swz_tr_base<DP>(lane, 1);
-    const float c2 = a.scale_log2;
-
-    auto compute = [&](const uint16_t* Qb, const uint16_t* Gb, const int buf, const int it) {
-      const uint32_t kq = opaque(kq0), t0 = opaque(trb0), t1 = opaque(trb1);
-      const bool is_self = it < G * n_self;
-      const int sq0 = is_self ? self_begin + (it % n_self) * BQ : 0;
-      // causal rows that end before the pair's first key contribute nothing
-      const bool skip = is_self && sq0 + BQ - 1 < wkey0;
-      const bool need_mask = (wkey0 + WKEYS > c_hi) || (is_self && sq0 < wkey0 + WKEYS - 1);
-      // ---- first half: S -> P (role P) or dP (role D)
-      const uint16_t* A1 = ROLE_P ? Qb : Gb;
-      f32x16_t sp[QB];
-      u16x8_t pk[QB][2];  // role P: P as the A operand of dV += P^T dO
-      u16x8_t pr[QB][2];  // role P: rounding residual of pk
-      if (!skip) {
-#pragma unroll
-        for (int qb = 0; qb < QB; ++qb) sp[qb] = zero16();
-        // operand reads run PF steps ahead of the MFMAs, in this order (the
-        // scheduling fences keep the compiler from sinking them)
-        {
-          constexpr int N1 = NKS * QB, PF = 6;
-          u16x8_t ring[PF];
-          auto rd = [&](int i) __attribute__((always_inline)) {
-            return lds8(A1, (i % QB) * 32 * DP * 2 + swz_b128<DP>(kq, i / QB));
-          };
-#pragma unroll
-          for (int i = 0; i < PF && i < N1; ++i) ring[i] = rd(i);
-#pragma unroll
-          for (int i = 0; i < N1; ++i) {
-            const u16x8_t x = ring[i % PF];
-            if (i + PF < N1) ring[i % PF] = rd(i + PF);
-            sp[i % QB] = mfma32<DT>(x, kv[i / QB], sp[i % QB]);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }
-        if constexpr (ROLE_P) {
-          auto to_p = [&](auto mask_tag) {
-            constexpr bool MASK = decltype(mask_tag)::value;
-#pragma unroll
-            for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                const int r0 = qb * 32 + 8 * j + 4 * hh;
-                const f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(&lse2s[buf][r0]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                  float p = fast_exp2(fmaf(sp[qb][4 * j + i], c2, -l4[i]));
-                  if constexpr (MASK)
-                    p = (mykey < c_hi && (!is_self || mykey <= sq0 + r0 + i)) ? p : 0.0f;
-                  const uint16_t hi = from_f32<DT>(p);
-                  pk[qb][j >> 1][(j & 1) * 4 + i] = hi;
-                  pr[qb][j >> 1][(j & 1) * 4 + i] = from_f32<DT>(p - to_f32<DT>(hi));
-                }
-              }
-          };
-          if (need_mask) to_p(std::true_type{}); else to_p(std::false_type{});
-#pragma unroll
-          for (int qb = 0; qb < QB; ++qb) {
-            Px[pair][qb][0][lane] = pk[qb][0];
-            Px[pair][qb][1][lane] = pk[qb][1];
-            Pr[pair][qb][0][lane] = pr[qb][0];
-            Pr[pair][qb][1][lane] = pr[qb][1];
-          }
-        }
-      }
-      lds_barrier();
-      // ---- second half: dV += P^T dO (role P) or dK += dS^T Q (role D)
-      if (!skip) {
-        u16x8_t op[QB][2];
-        if constexpr (ROLE_P) {
-#pragma unroll
-          for (int qb = 0; qb < QB; ++qb) { op[qb][0] = pk[qb][0]; op[qb][1] = pk[qb][1]; }
-        } else {
-#pragma unroll
-          for (int qb = 0; qb < QB; ++qb) {
-            const u16x8_t px[2] = {Px[pair][qb][0][lane], Px[pair][qb][1][lane]};
-            const u16x8_t rx[2] = {Pr[pair][qb][0][lane], Pr[pair][qb][1][lane]};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const f32x4_t d4 =
-                  *reinterpret_cast<const f32x4_t*>(&dels[buf][qb * 32 + 8 * j + 4 * hh]);
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                const int r = 4 * j + i, h2 = j >> 1, x = (j & 1) * 4 + i;
-                const float pv = to_f32<DT>(px[h2][x]) + to_f32<DT>(rx[h2][x]);
-                op[qb][h2][x] = from_f32<DT>(pv * (sp[qb][r] - d4[i]));
-              }
-            }
-          }
-        }
-        const uint16_t* B2 = ROLE_P ? Gb : Qb;
-        {
-          constexpr int N2 = NDB * QB * 2, PF = 6;
-          u16x8_t ring[PF];
-          // step i: d block i / (2 QB), row block (i / 2) % QB, half i % 2
-          auto rd = [&](int i) __attribute__((always_inline)) {
-            const uint32_t ro = (((i / 2) % QB) * 32 + (i % 2) * 16) * DP * 2;
-            const int db = i / (2 * QB);
-            return lds_tr8(B2, ro + swz_tr<DP>(t0, db), ro + swz_tr<DP>(t1, db));
-          };
-#pragma unroll
-          for (int i = 0; i < PF && i < N2; ++i) ring[i] = rd(i);
-#pragma unroll
-          for (int i = 0; i < N2; ++i) {
-            const u16x8_t b = ring[i % PF];
-            if (i + PF < N2) ring[i % PF] = rd(i + PF);
-            acc[i / (2 * QB)] = mfma32<DT>(op[(i / 2) % QB][i % 2], b, acc[i / (2 * QB)]);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }
-      }
-    };
-
-    if (it_lo < it_hi) {
-      fetch_rows(it_lo);
-      load_ld();
-      dma(Q0, G0);
-      store_ld(0);
-      fetch_rows(it_lo + 1);
-    }
-    stage_barrier();
-    for (int it = it_lo; it < it_hi; it += 2) {
-      if (it + 1 < it_hi) {
-        load_ld();
-        dma(Q1, G1);
-        fetch_rows(it + 2);
-      }
-      compute(Q0, G0, 0, it);
-      if (it + 1 < it_hi) store_ld(1);
-      stage_barrier();
-      if (it + 1 >= it_hi) break;
-      if (it + 2 < it_hi) {
-        load_ld();
-        dma(Q0, G0);
-        fetch_rows(it + 3);
-      }
-      compute(Q1, G1, 1, it + 1);
-      if (it + 2 < it_hi) store_ld(0);
-      stage_barrier();
-    }
-
-    // D-layout: lane holds column d = i*32 + qi, keys 8j + 4hh + r.  A row
-    // split writes fp32 partials to its slot for the fixed-order reduction.
-    if (slot >= 0) {
-      float* pdst = a.part_dkv + (int64_t)slot * kv_slot_floats(D) + (ROLE_P ? kKvTileKeys * D : 0);
-#pragma unroll
-      for (int i = 0; i < NDB; ++i) {
-        const int d = i * 32 + qi;
-        if (d >= D) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = wkey0 + 8 * (r >> 2) + 4 * hh + (r & 3);
-          if (key < c_hi) pdst[(key - key0) * D + d] = acc[i][r];
-        }
-      }
-      return;
-    }
-    uint16_t* dst = ROLE_P ? a.dv : a.dk;
-    const float osc = ROLE_P ? 1.0f : a.scale;
-#pragma unroll
-    for (int i = 0; i < NDB; ++i) {
-      const int d = i * 32 + qi;
-      if (d >= D) continue;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = wkey0 + 8 * (r >> 2) + 4 * hh + (r & 3);
-        if (key < c_hi) dst[((int64_t)key * a.Hkv + kh) * D + d] = from_f32<DT>(acc[i][r] * osc);
-      }
-    }
-  };
-  if (role_p) body(std::true_type{}); else body(std::false_type{});
-}
-
 // Row-split schedule of the key-major kernels, built on the device because
 // the expert row counts live there.  Tile t costs n_t row tiles (its causal
 // tiles for the G heads plus its expert's packed tiles, the count every
@@ -932,7 +615,7 @@ int launch_bwd(const BwdArgs& a, int n_self, int n_kv, int max_remote, int parts
       if constexpr (DP <= 64) launch_dkdv1<DT, DP>(a, n_wg, st);
       else launch_dkdv2<DT, DP>(a, n_wg, st);
     } else {
-      hipLaunchKernelGGL((dkdv_kernel<DT, DP>), dim3(n_wg), dim3(512), 0, st, a);
+      launch_dkdv4<DT, DP>(a, n_wg, st);
     }
     if (a.kv_splits > 1)
       hipLaunchKernelGGL(dkdv_reduce_kernel<DT>, dim3(n_kv, kReduceSplit), dim3(256), 0, st, a);

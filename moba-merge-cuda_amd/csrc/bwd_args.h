@@ -60,8 +60,11 @@ struct BwdArgs {
 // or, with a row-split schedule, one per schedule entry.
 // dkdv1 (attn_dkdv.hip): all four products per wave, head dims <= 64.
 // dkdv2 (attn_dkdv2.hip): wave pairs with split roles, head dims 65..128.
+// dkdv4 (attn_dkdv4.hip): wave pairs with split roles, 32-row tiles, expert
+// rows gathered, head dims 129..256.
 template <int DT, int DP> void launch_dkdv1(const BwdArgs& a, int n_wg, hipStream_t st);
 template <int DT, int DP> void launch_dkdv2(const BwdArgs& a, int n_wg, hipStream_t st);
+template <int DT, int DP> void launch_dkdv4(const BwdArgs& a, int n_wg, hipStream_t st);
 
 // Keys per dK/dV workgroup (every key-major kernel) and the size of one
 // partial slot in floats.

@@ -89,8 +89,12 @@ class PrefillPlan:
         # few kv heads leave too few key tiles to fill the chip: split each
         # tile's query rows over several workgroups (fp32 partials + reduce);
         # about 1536 workgroups in all (cfg2: 6 splits, 1.50-1.52 ms per step
-        # against 1.53 with 4 and 8, 1.54-1.58 with 12-16)
-        self.kv_splits = (max(1, min(8, 1536 // max(1, self.n_kv_tiles)))
+        # against 1.53 with 4 and 8, 1.54-1.58 with 12-16); half of that above
+        # 128 dims, where a slot is twice as large (T 8192, 16/4 heads, D 256:
+        # dK/dV kernel and reduction 730 + 48 us with 768, 707 + 68 with 1024,
+        # 742 + 32 with 512)
+        wgs = 1536 if head_dim <= 128 else 768
+        self.kv_splits = (max(1, min(8, wgs // max(1, self.n_kv_tiles)))
                           if head_dim % 8 == 0 else 1)
         kv_flat = self.kv_tiles_list
 
