@@ -392,51 +392,14 @@ MOBA_DEV float wave_sum(float v) {
 }
 
 
-// acc = fma(b_j, m[j], acc) for j = 0..7 in order, b_j = lane (row base + J0
-// + j) of b: the fma reads b through a DPP row broadcast (row_newbcast, one
-// source lane for each 16-lane row), which the compiler does not form on its
-// own.  A 16-lane row then holds 16 dims of a row vector in one register, and
-// a whole wave streams a sequential fma chain against it with no LDS reads.
-// The leading s_nop covers the DPP read-after-VALU-write hazard on b (the
-// compiler does not look inside the block).
-template <int J0>
-MOBA_DEV float fma8_bcast(float acc, float b, const float (&m)[8]) {
-  static_assert(J0 == 0 || J0 == 8, "row lanes 0..7 or 8..15");
-  if constexpr (J0 == 0) {
-    asm volatile(
-        "s_nop 1\n"
-        "v_fmac_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %3 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %4 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %5 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %6 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %7 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %8 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %9 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
-        : "+v"(acc)
-        : "v"(b), "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "v"(m[5]), "v"(m[6]),
-          "v"(m[7]));
-  } else {
-    asm volatile(
-        "s_nop 1\n"
-        "v_fmac_f32_dpp %0, %1, %2 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %3 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %4 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %5 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %6 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %7 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %8 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %9 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
-        : "+v"(acc)
-        : "v"(b), "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "v"(m[5]), "v"(m[6]),
-          "v"(m[7]));
-  }
-  return acc;
-}
-
-// Four chains interleaved: acc[k] = fma(lane (row base + J0 + j) of b[k],
-// m[j], acc[k]) for j = 0..7 in order, chain k independent of the others (so
-// consecutive instructions do not wait on each other).  Hazard as above.
+// acc[k] = fma(lane (row base + J0 + j) of b[k], m[j], acc[k]) for j = 0..7 in
+// order, four independent chains k interleaved (so consecutive instructions
+// do not wait on each other).  The fma reads b through a DPP row broadcast
+// (row_newbcast, one source lane for each 16-lane row), which the compiler
+// does not form on its own: a 16-lane row then holds 16 dims of a row vector
+// in one register, and a whole wave streams sequential fma chains against it
+// with no LDS reads.  The leading s_nop covers the DPP read-after-VALU-write
+// hazard on b (the compiler does not look inside the block).
 #define MOBA_F4(J, MJ)                                                                         \
   "v_fmac_f32_dpp %0, %4, " MJ " row_newbcast:" #J " row_mask:0xf bank_mask:0xf\n"             \
   "v_fmac_f32_dpp %1, %5, " MJ " row_newbcast:" #J " row_mask:0xf bank_mask:0xf\n"             \

@@ -10,6 +10,8 @@
 //           input dtype: route_precision "upstream")
 //   gate  = fma chain over d = 0..D-1 in fp32
 //   top-k = descending gate, exact ties -> lowest chunk, -inf never chosen.
+#include <type_traits>
+
 #include "common.h"
 #include "../../include/moba_hip.h"
 
@@ -113,20 +115,55 @@ __global__ __launch_bounds__(256) void chunk_means_kernel(const uint16_t* __rest
 
 // One thread per (token, q head): a workgroup takes 256 consecutive tokens of
 // one head.  The means rows its tokens score (filtered indices [flo, fhi) of
-// the head's kv head) go through LDS in tiles of kRouteTile rows.  A wave
-// walks the union of its lanes' candidate ranges in a wave-uniform loop:
-// each 16-lane row of the wave reads 16 values of the candidate's means row
-// into one register per 16 dims, and the fma chain takes dim d from lane
-// d % 16 of its row by a DPP row broadcast (an operand modifier of the fma),
-// so a means row costs DP / 16 LDS reads per wave instead of DP / 4
-// broadcast 16-byte reads; lanes outside a candidate's range discard its
-// score.  The token's q row is held in registers (fp32 up to 128 dims, the
-// input dtype above).  The fma chain of each candidate is the canonical
-// order, unchanged.
+// the head's kv head) go through LDS in tiles of kRouteTile rows; a wave walks
+// the union of its lanes' candidate ranges, 16 or 8 candidates at a time, and
+// lanes outside a candidate's range discard its score.
+//
+// The canonical gate is a sequential fma chain over d per (token, candidate):
+// too long for the vector unit (each fma also needs the candidate's mean in
+// every lane), but it is what v_mfma_f32_4x4x1_16b_f32 does: one fma per
+// output, 16 blocks of 4 candidates x 4 tokens, so D of them in d order form
+// the chains of 4 candidates for the wave's 64 tokens, bit for bit, at twice
+// the rate of plain fmas.  Lane l supplies its token's q[d] and the mean of
+// candidate l % 4, and receives its own token's four scores.  Rows of the LDS
+// tile are padded by 16 bytes, so the four rows a read touches lie in
+// different banks; the token's q row stays in the input type (half the
+// registers, converted as it is used).  Against a chain of fmas with the mean
+// in a DPP row broadcast (T 32768, 8 heads, D 128, 63 candidates: 138 -> 87
+// us; 32 heads, 7 candidates: 116 -> 97; T 8192, 16 heads, D 256, 7
+// candidates: 43 -> 24).  Eight candidates a pass instead of 16 took 101 us
+// in the first case (the conversions), four 117.
 constexpr int kRouteTile = 32;
 
-// DE: the head dim when it is DP exactly (no per-piece bound checks), else 0.
-template <int DT, int DP, int DE>
+// The four values of two packed words, converted where they are used: kept
+// out of the compiler's sight, which would convert the whole row ahead of the
+// loop and hold it in twice the registers.  The trailing s_nop covers the two
+// wait states between a vector write and an MFMA that reads it (the compiler
+// does not look inside the block).
+template <int DT> MOBA_DEV f32x4_t late_f32x4(uint32_t w0, uint32_t w1) {
+  float x0, x1, x2, x3;
+  if constexpr (DT == 0) {
+    asm volatile(
+        "v_lshlrev_b32 %0, 16, %4\n"
+        "v_and_b32 %1, 0xffff0000, %4\n"
+        "v_lshlrev_b32 %2, 16, %5\n"
+        "v_and_b32 %3, 0xffff0000, %5\n"
+        "s_nop 1"
+        : "=&v"(x0), "=&v"(x1), "=&v"(x2), "=&v"(x3) : "v"(w0), "v"(w1));
+  } else {
+    asm volatile(
+        "v_cvt_f32_f16 %0, %4\n"
+        "v_cvt_f32_f16_sdwa %1, %4 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1\n"
+        "v_cvt_f32_f16 %2, %5\n"
+        "v_cvt_f32_f16_sdwa %3, %5 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1\n"
+        "s_nop 1"
+        : "=&v"(x0), "=&v"(x1), "=&v"(x2), "=&v"(x3) : "v"(w0), "v"(w1));
+  }
+  return (f32x4_t){x0, x1, x2, x3};
+}
+
+// RM: the largest R the selection registers hold.
+template <int DT, int DP, int RM>
 __global__ __launch_bounds__(256) void route_kernel(const uint16_t* __restrict__ q, int T, int Hq,
                                                     int Hkv, int D,
                                                     const float* __restrict__ means,
@@ -136,19 +173,47 @@ __global__ __launch_bounds__(256) void route_kernel(const uint16_t* __restrict__
                                                     int F, int* __restrict__ sel,
                                                     float* __restrict__ gate,
                                                     int* __restrict__ blk_count) {
-  __shared__ __attribute__((aligned(16))) float mt[kRouteTile * DP];
+  constexpr int LD = DP + 4;  // floats per LDS row of the means tile
+  // 256 tokens x 64 dims of q while it is loaded, then the means tiles
+  constexpr int kStageFloats = 256 * 64 / 2;
+  __shared__ __attribute__((aligned(16))) float mt[kRouteTile * LD > kStageFloats ? kRouteTile * LD : kStageFloats];
   __shared__ int red[2][4];
   const int tid = threadIdx.x, lane = tid & 63;
   const int s = blockIdx.x * 256 + tid;
   const int h = blockIdx.y;
   const bool live = s < T;
   const int G = Hq / Hkv, kh = h / G;
-  // the q row first: its loads overlap the chunk search below
+  // The wave's q rows come in whole 128-byte lines, 8 lanes to a row of 64
+  // dims, and reach their lanes through LDS (16-byte block x of row r at block
+  // x ^ (r / 2 % 8): no bank conflicts either way).  Each lane loading its own
+  // row took eight times the lines.
   const int64_t idx = (int64_t)s * Hq + h;
   constexpr int NQ = DP / 8;
   u16x8_t qv[NQ];
+  {
+    uint16_t* st = reinterpret_cast<uint16_t*>(mt) + (tid >> 6) * 64 * 64;
+    const int s0 = blockIdx.x * 256 + (tid >> 6) * 64;
+    u16x8_t x[NQ];
 #pragma unroll
-  for (int i = 0; i < NQ; ++i) qv[i] = (live && i * 8 < D) ? ld8(q + idx * D + i * 8) : zero8();
+    for (int i = 0; i < NQ; ++i) {  // slice i / 8 of 64 dims, rows 8 (i % 8) ..
+      const int r = (i % 8) * 8 + (lane >> 3), d = (i / 8) * 64 + (lane & 7) * 8;
+      x[i] = ld8(q + ((int64_t)min(s0 + r, T - 1) * Hq + h) * D + (d < D ? d : 0));
+      if (d >= D) x[i] = zero8();
+    }
+#pragma unroll
+    for (int sl = 0; sl < NQ / 8; ++sl) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = i * 8 + (lane >> 3);
+        st8(st + r * 64 + (((lane & 7) ^ ((r >> 1) & 7)) * 8), x[sl * 8 + i]);
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        qv[sl * 8 + i] = ld8(st + lane * 64 + ((i ^ ((lane >> 1) & 7)) * 8));
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
   // chunk containing s (the last token's for the threads past T)
   const int sc = live ? s : T - 1;
   // search once per wave for its first token (uniform loads), then per lane
@@ -181,25 +246,15 @@ __global__ __launch_bounds__(256) void route_kernel(const uint16_t* __restrict__
   const int flo = min(min(red[0][0], red[0][1]), min(red[0][2], red[0][3]));
   const int fhi = max(max(red[1][0], red[1][1]), max(red[1][2], red[1][3]));
 
-  constexpr bool QF32 = DP <= 128;      // q row as fp32 registers
-  float qf[QF32 ? DP : 1];
-  if constexpr (QF32) {
-#pragma unroll
-    for (int i = 0; i < NQ; ++i)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) qf[i * 8 + e] = to_f32<DT>(qv[i][e]);
-  }
-
-  float val[kMaxRemote];
-  int ix[kMaxRemote];
+  float val[RM];
+  int ix[RM];
   int cnt = 0;
 #pragma unroll
-  for (int j = 0; j < kMaxRemote; ++j) { val[j] = -INFINITY; ix[j] = -1; }
+  for (int j = 0; j < RM; ++j) { val[j] = -INFINITY; ix[j] = -1; }
 
-  // LDS tile: rows of DP floats, columns past D zero (so are q's), and
-  // fma(0, 0, acc) == acc keeps the chain exact over the padding
+  // LDS tile: columns past D and rows past the tile's end zero (so are q's),
+  // and fma(0, 0, acc) == acc keeps the chain exact over the padding
   constexpr int NST = (kRouteTile * DP / 4 + 255) / 256;
-  constexpr int NM = DP / 16;  // registers of a means row per lane
   for (int t0 = flo; t0 < fhi; t0 += kRouteTile) {
     const int nt = min(kRouteTile, fhi - t0);
     f32x4_t stg[NST];
@@ -214,51 +269,66 @@ __global__ __launch_bounds__(256) void route_kernel(const uint16_t* __restrict__
 #pragma unroll
     for (int i = 0; i < NST; ++i) {
       const int x = tid + 256 * i;
-      if (x < kRouteTile * DP / 4) *reinterpret_cast<f32x4_t*>(mt + x * 4) = stg[i];
+      if (x < kRouteTile * DP / 4)
+        *reinterpret_cast<f32x4_t*>(mt + (x / (DP / 4)) * LD + (x % (DP / 4)) * 4) = stg[i];
     }
     __syncthreads();
     const int fa = max(wlo, t0), fb = min(whi, t0 + nt);
-    for (int f = fa; f < fb; ++f) {
-      const float* mr = mt + (f - t0) * DP + (lane & 15);
-      float mv[NM];
+    // 4 NC candidates from g on, NC independent chains per lane; rows past the
+    // tile are read as its last and their scores discarded
+    auto group = [&](int g, auto nc_tag) __attribute__((always_inline)) {
+      constexpr int NC = decltype(nc_tag)::value;
+      const float* row[NC];
+      f32x4_t acc[NC];
 #pragma unroll
-      for (int i = 0; i < NM; ++i) mv[i] = mr[16 * i];
-      // sequential fma chain over d = 0 .. DP-1 (zero past D)
-      float acc = 0.0f;
-#pragma unroll
-      for (int i = 0; i < NM; ++i) {
-        float qa[8], qb[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          qa[e] = QF32 ? qf[16 * i + e] : to_f32<DT>(qv[2 * i][e]);
-          qb[e] = QF32 ? qf[16 * i + 8 + e] : to_f32<DT>(qv[2 * i + 1][e]);
-        }
-        acc = fma8_bcast<0>(acc, mv[i], qa);
-        acc = fma8_bcast<8>(acc, mv[i], qb);
+      for (int k = 0; k < NC; ++k) {
+        row[k] = mt + min(g - t0 + 4 * k + (lane & 3), kRouteTile - 1) * LD;
+        acc[k] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
       }
-      if (!(live && f >= f0 && f < f1)) continue;
-      const int c = f + b;
-      if (gate) gate[((int64_t)f * Hq + h) * T + s] = acc;
-      // stable insertion into the descending list: equal scores stay behind the
-      // earlier (lower) chunk, so exact ties resolve to the lowest index.
-      if (cnt == R && !(acc > val[R - 1])) continue;
-      int pos = 0;
 #pragma unroll
-      for (int j = 0; j < kMaxRemote; ++j) pos += (j < cnt && val[j] >= acc);
+      for (int d4 = 0; d4 < DP / 4; ++d4) {
+        f32x4_t m[NC];
 #pragma unroll
-      for (int j = kMaxRemote - 1; j >= 1; --j)
-        if (j > pos && j < R) { val[j] = val[j - 1]; ix[j] = ix[j - 1]; }
+        for (int k = 0; k < NC; ++k) m[k] = *reinterpret_cast<const f32x4_t*>(row[k] + 4 * d4);
+        const u32x4_t w = __builtin_bit_cast(u32x4_t, qv[d4 / 2]);
+        const f32x4_t x = late_f32x4<DT>(w[(d4 % 2) * 2], w[(d4 % 2) * 2 + 1]);
 #pragma unroll
-      for (int j = 0; j < kMaxRemote; ++j)
-        if (j == pos) { val[j] = acc; ix[j] = c; }
-      if (cnt < R) cnt++;
-    }
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int k = 0; k < NC; ++k)
+            acc[k] = __builtin_amdgcn_mfma_f32_4x4x1f32(m[k][e], x[e], acc[k], 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4 * NC; ++r) {
+        const int f = g + r;
+        const float score = acc[r / 4][r % 4];
+        if (f >= fb || !(live && f >= f0 && f < f1)) continue;
+        const int c = f + b;
+        if (gate) gate[((int64_t)f * Hq + h) * T + s] = score;
+        // stable insertion into the descending list: equal scores stay behind the
+        // earlier (lower) chunk, so exact ties resolve to the lowest index.
+        if (cnt == R && !(score > val[R - 1])) continue;
+        int pos = 0;
+#pragma unroll
+        for (int j = 0; j < RM; ++j) pos += (j < cnt && val[j] >= score);
+#pragma unroll
+        for (int j = RM - 1; j >= 1; --j)
+          if (j > pos && j < R) { val[j] = val[j - 1]; ix[j] = ix[j - 1]; }
+#pragma unroll
+        for (int j = 0; j < RM; ++j)
+          if (j == pos) { val[j] = score; ix[j] = c; }
+        if (cnt < R) cnt++;
+      }
+    };
+    int g = fa;
+    for (; fb - g > 8; g += 16) group(g, std::integral_constant<int, 4>{});
+    for (; g < fb; g += 8) group(g, std::integral_constant<int, 2>{});
   }
   // ascending chunk order for the slot list (static sorting network)
 #pragma unroll
-  for (int pass = 0; pass < kMaxRemote; ++pass) {
+  for (int pass = 0; pass < RM; ++pass) {
 #pragma unroll
-    for (int j = 0; j + 1 < kMaxRemote; ++j) {
+    for (int j = 0; j + 1 < RM; ++j) {
       if (j + 1 < cnt && ix[j] > ix[j + 1]) { int t = ix[j]; ix[j] = ix[j + 1]; ix[j + 1] = t; }
     }
   }
@@ -270,8 +340,8 @@ __global__ __launch_bounds__(256) void route_kernel(const uint16_t* __restrict__
   // this workgroup's count of every candidate, for the expert packing
   int fs[kMaxRemote];
 #pragma unroll
-  for (int j = 0; j < kMaxRemote; ++j) fs[j] = live && j < cnt ? ix[j] - b : -1;
-  static_assert(kRouteTile * DP * 4 >= kPickRows * 4 * 8, "the means tile holds the pick bits");
+  for (int j = 0; j < kMaxRemote; ++j) fs[j] = live && j < RM && j < cnt ? ix[j < RM ? j : 0] - b : -1;
+  static_assert(sizeof(mt) >= kPickRows * 4 * 8, "the means tile holds the pick bits");
   uint64_t* bits = reinterpret_cast<uint64_t*>(mt);
   int* dst = blk_count + (int64_t)h * gridDim.x + blockIdx.x;
   const int64_t fstep = (int64_t)Hq * gridDim.x;
@@ -582,19 +652,21 @@ static int route_prefill(const void* q, int dtype, int T, int Hq, int Hkv, int D
   if (D > 256) { moba_set_error("route_prefill: head_dim must be at most 256"); return MOBA_ERR_ARG; }
   dim3 grid((unsigned)((T + 255) / 256), (unsigned)Hq), block(256);
   const uint16_t* qp = (const uint16_t*)q;
-#define MOBA_ROUTE(DT_, DP_, DE_) \
-  hipLaunchKernelGGL((route_kernel<DT_, DP_, DE_>), grid, block, 0, st, qp, T, Hq, Hkv, D, means, \
+#define MOBA_ROUTE(DT_, DP_, RM_) \
+  hipLaunchKernelGGL((route_kernel<DT_, DP_, RM_>), grid, block, 0, st, qp, T, Hq, Hkv, D, means, \
                      cu_chunk, nchunk, chunk_batch, first_chunk, R, F, sel, gate, blk_count)
+#define MOBA_ROUTE_RM(DT_, DP_) \
+  if (R <= 4) MOBA_ROUTE(DT_, DP_, 4); else MOBA_ROUTE(DT_, DP_, 8);
 #define MOBA_ROUTE_DT(DT_) \
-  if (D == 64) MOBA_ROUTE(DT_, 64, 64); else if (D < 64) MOBA_ROUTE(DT_, 64, 0); \
-  else if (D == 128) MOBA_ROUTE(DT_, 128, 128); else if (D < 128) MOBA_ROUTE(DT_, 128, 0); \
-  else if (D == 256) MOBA_ROUTE(DT_, 256, 256); else MOBA_ROUTE(DT_, 256, 0);
+  if (D <= 64) { MOBA_ROUTE_RM(DT_, 64) } else if (D <= 128) { MOBA_ROUTE_RM(DT_, 128) } \
+  else { MOBA_ROUTE_RM(DT_, 256) }
   if (dtype == 0) {
     MOBA_ROUTE_DT(0)
   } else {
     MOBA_ROUTE_DT(1)
   }
 #undef MOBA_ROUTE_DT
+#undef MOBA_ROUTE_RM
 #undef MOBA_ROUTE
   return moba_launch_status("route_prefill");
 }

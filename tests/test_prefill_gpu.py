@@ -488,3 +488,26 @@ def test_remote_tiles_given_or_searched(cuda_device, monkeypatch, hq, hkv, dim, 
     monkeypatch.setattr(P._lib, "call", searched)
     for a, b in zip(given, grads()):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dim", [40, 64, 128, 136, 256])
+@pytest.mark.parametrize("topk", [3, 9])
+@pytest.mark.parametrize("scale", [1e-20, 3e18])
+def test_gate_bits_at_the_ends_of_the_range(cuda_device, dim, topk, scale):
+    """Gate chains whose products and sums are subnormal in fp32, and ones that
+    overflow on the way: every score has the oracle's bits, for both widths of
+    the selection registers, with more candidates than one 16-wide pass and
+    tokens on both sides of a 256-token block."""
+    q, k, v, cu, ml, _ = prefill_inputs(4, 2, dim, (300, 37), torch.bfloat16, seed=31)
+    q, k = q.detach() * scale, k.detach() * scale
+    plan, rt, gate = _gpu_route(q, k, cu, {"chunk_size": 11, "topk": topk}, 1)
+    sel, means, gate_ref, _ = oracle_route(q, k, cu, 11, topk, 1)
+    np.testing.assert_array_equal(rt.means.cpu().numpy().view(np.uint32), means.view(np.uint32))
+    g = gate.cpu().numpy()
+    nan = np.isnan(gate_ref)
+    np.testing.assert_array_equal(np.isnan(g), nan)
+    np.testing.assert_array_equal(g[~nan].view(np.uint32), gate_ref[~nan].view(np.uint32))
+    tiny = np.abs(gate_ref[~nan & np.isfinite(gate_ref)])
+    assert scale > 1 or ((tiny > 0) & (tiny < 2.0 ** -126)).any()
+    if not nan.any():
+        np.testing.assert_array_equal(rt.sel.cpu().numpy(), sel)
