@@ -141,5 +141,6 @@ def ptr(t) -> int | None:
 
 
 def stream_of(device) -> int:
+    """Raw handle of the current stream of a tensor's device."""
     import torch
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)

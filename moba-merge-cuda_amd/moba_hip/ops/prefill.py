@@ -8,6 +8,7 @@ by tensor object (lru_cache, diagnostic.py:30).
 """
 from __future__ import annotations
 
+import math
 import threading
 from collections import OrderedDict
 
@@ -30,6 +31,29 @@ def attn_rows(head_dim):
 def dkdv_keys(head_dim):
     """Keys per dK/dV workgroup: 4 wave pairs x 32 keys."""
     return 128
+
+
+class Layout:
+    """Named arrays in one allocation, each 256-byte aligned."""
+
+    def __init__(self, **arrays):
+        self.at, self.nbytes = {}, 0
+        for name, (dtype, shape) in arrays.items():
+            n = math.prod(shape) * dtype.itemsize
+            self.at[name] = (self.nbytes, n, dtype, shape)
+            self.nbytes += -(-n // 256) * 256
+
+    def alloc(self, device):
+        return torch.empty(self.nbytes, dtype=torch.uint8, device=device)
+
+    def ptrs(self, buf):
+        """Address of every array in ``buf`` (None for an empty one)."""
+        base = buf.data_ptr()
+        return {name: base + at if n else None for name, (at, n, _, _) in self.at.items()}
+
+    def view(self, buf, name):
+        at, n, dtype, shape = self.at[name]
+        return buf[at:at + n].view(dtype).view(shape)
 
 
 class PrefillPlan:
@@ -107,6 +131,36 @@ class PrefillPlan:
             self._views[name] = (len(flat), len(vals))
             flat.extend(vals)
         self.meta = torch.tensor(flat, dtype=torch.int32).to(device, non_blocking=False)
+        base = self.meta.data_ptr()
+        self._ptrs = {name: base + 4 * off for name, (off, _) in self._views.items()}
+        self._workspaces()
+
+    def _workspaces(self):
+        """Layouts of the workspaces of one call, each one allocation (an
+        allocation costs the host about 2 us): what the forward leaves for the
+        backward, and what each of the two needs while it runs."""
+        T, hq, hkv, d = self.cu[-1], self.hq, self.hkv, self.head_dim
+        F, R, E, lib = self.num_filtered, self.remote, self.num_experts, _lib.load()
+        slots = T * hq * R
+        self.n_tile_slots = -(-self.max_remote_tiles // 8) * 8
+        self.routing = Layout(
+            means=(torch.float32, (F, hkv, d)), sel=(torch.int32, (T, hq, R)),
+            counts=(torch.int32, (E,)), row_off=(torch.int32, (E + 1,)),
+            tile_off=(torch.int32, (E + 1,)), rows=(torch.int32, (max(1, slots),)),
+            tiles=(torch.int32, (self.n_tile_slots, 4)))
+        self.route_work = Layout(work=(torch.int32, (
+            max(1, lib.moba_hip_pack_experts_work(T, hq, hkv, F)),)))
+        self.fwd_work = Layout(part_o=(torch.bfloat16, (slots, d)),   # either 16-bit type
+                               part_ml=(torch.float32, (slots, 2)))
+        # row-split workspace: the device-built schedule, then fp32 partial
+        # slots; pack: expert rows of q / dO / lse / delta, contiguous for the
+        # key-major kernels
+        split = (lib.moba_hip_prefill_bwd_work(self.n_kv_tiles, self.kv_splits, d)
+                 if self.kv_splits > 1 else 0)
+        self.bwd_work = Layout(
+            delta=(torch.float32, (2, T * hq)), part_dq=(torch.bfloat16, (slots, d)),
+            part_dkv=(torch.uint8, (split,)),
+            pack=(torch.uint8, (slots * (4 * d + 8) if d <= 128 else 0,)))
 
     N_XCD = 8  # workgroup L of a 1-D grid runs on XCD L % 8
 
@@ -189,7 +243,7 @@ class PrefillPlan:
         return self.meta[off:off + n]
 
     def ptr(self, name):
-        return self.dev(name).data_ptr()
+        return self._ptrs[name]
 
 
 _PLANS: "OrderedDict[tuple, PrefillPlan]" = OrderedDict()
@@ -215,8 +269,21 @@ def get_plan(cu, chunk, hq, hkv, head_dim, topk, device, fallback=False):
 
 
 class RouteResult:
-    """Device routing state shared by the forward and the backward."""
-    __slots__ = ("sel", "counts", "row_off", "tile_off", "rows", "tiles", "means")
+    """Device routing state shared by the forward and the backward: ``means``,
+    ``sel``, ``counts``, ``row_off``, ``tile_off``, ``rows`` and ``tiles`` in
+    one buffer (``ptr`` holds their addresses; as attributes they are views)."""
+
+    def __init__(self, plan=None, device=None):
+        if plan is not None:
+            self.layout = plan.routing
+            self.buf = plan.routing.alloc(device)
+            self.ptr = plan.routing.ptrs(self.buf)
+
+    def __getattr__(self, name):
+        layout = self.__dict__.get("layout")
+        if layout is None or name not in layout.at:
+            raise AttributeError(name)
+        return layout.view(self.buf, name)
 
 
 def route(plan: PrefillPlan, q, k, precision: int, want_gate=False):
@@ -224,28 +291,21 @@ def route(plan: PrefillPlan, q, k, precision: int, want_gate=False):
     (and the masked gate [F,Hq,T] when ``want_gate``)."""
     T, hq, d = q.shape
     dev = q.device
-    st = _lib.stream_of(dev)
-    code = DTYPE_CODE[q.dtype]
-    r = RouteResult()
-    F, R, E = plan.num_filtered, plan.remote, plan.num_experts
-    r.means = torch.empty((F, plan.hkv, d), dtype=torch.float32, device=dev)
-    r.sel = torch.empty((T, hq, R), dtype=torch.int32, device=dev)
-    r.counts = torch.empty(E, dtype=torch.int32, device=dev)
-    r.row_off = torch.empty(E + 1, dtype=torch.int32, device=dev)
-    r.tile_off = torch.empty(E + 1, dtype=torch.int32, device=dev)
-    r.rows = torch.empty(max(1, T * hq * R), dtype=torch.int32, device=dev)
-    r.tiles = torch.empty((-(-plan.max_remote_tiles // 8) * 8, 4), dtype=torch.int32, device=dev)
+    F, R = plan.num_filtered, plan.remote
+    r = RouteResult(plan, dev)
     gate = torch.empty((F, hq, T), dtype=torch.float32, device=dev) if want_gate else None
-    work = torch.empty(max(1, _lib.load().moba_hip_pack_experts_work(T, hq, plan.hkv, F)),
-                       dtype=torch.int32, device=dev)
-    _lib.call("moba_hip_prefill_route", q.data_ptr(), k.data_ptr(), code, T, hq, plan.hkv, d,
-              plan.ptr("chunk_start"), plan.chunk, precision, plan.ptr("cu_chunk"),
-              len(plan.chunk_batch), plan.ptr("chunk_batch"), plan.ptr("first_chunk"),
-              plan.ptr("cu_seqlens"), plan.ptr("filtered"), R, F, plan.block_rows,
-              r.means.data_ptr(), r.sel.data_ptr(), _lib.ptr(gate), r.counts.data_ptr(),
-              r.row_off.data_ptr(), r.tile_off.data_ptr(), r.rows.data_ptr(), r.tiles.data_ptr(),
-              r.tiles.shape[0], work.data_ptr(), st)
+    work = plan.route_work.alloc(dev)
+    at, ptr = r.ptr, plan._ptrs
+    _lib.call("moba_hip_prefill_route", q.data_ptr(), k.data_ptr(), DTYPE_CODE[q.dtype], T, hq,
+              plan.hkv, d, ptr["chunk_start"], plan.chunk, precision, ptr["cu_chunk"],
+              len(plan.chunk_batch), ptr["chunk_batch"], ptr["first_chunk"], ptr["cu_seqlens"],
+              ptr["filtered"], R, F, plan.block_rows, at["means"], at["sel"], _lib.ptr(gate),
+              at["counts"], at["row_off"], at["tile_off"], at["rows"], at["tiles"],
+              plan.n_tile_slots, work.data_ptr(), _lib.stream_of(dev))
     return (r, gate) if want_gate else r
+
+
+_NO_ROUTE = dict.fromkeys(("sel", "counts", "row_off", "tile_off", "rows", "tiles"))
 
 
 def forward(plan: PrefillPlan, q, k, v, rt: RouteResult | None):
@@ -255,19 +315,15 @@ def forward(plan: PrefillPlan, q, k, v, rt: RouteResult | None):
     R = plan.remote
     out = torch.empty_like(q)
     lse = torch.empty((T, hq), dtype=torch.float32, device=dev)
-    part_o = part_ml = None
-    if R:
-        part_o = torch.empty((T * hq * R, d), dtype=q.dtype, device=dev)
-        part_ml = torch.empty((T * hq * R, 2), dtype=torch.float32, device=dev)
+    buf = plan.fwd_work.alloc(dev) if R else None
+    work = plan.fwd_work.ptrs(buf) if R else {"part_o": None, "part_ml": None}
+    at, ptr = rt.ptr if R else _NO_ROUTE, plan._ptrs
     _lib.call("moba_hip_prefill_fwd_tiles", q.data_ptr(), k.data_ptr(), v.data_ptr(),
               DTYPE_CODE[q.dtype], T, hq, plan.hkv, d, d ** -0.5,
-              plan.ptr("att_chunk"), plan.ptr("self_tiles"), plan.n_self_tiles,
-              _lib.ptr(rt.sel) if R else None, R, plan.ptr("filtered"), plan.num_experts,
-              _lib.ptr(rt.tile_off) if R else None, _lib.ptr(rt.row_off) if R else None,
-              _lib.ptr(rt.counts) if R else None, _lib.ptr(rt.rows) if R else None,
-              _lib.ptr(rt.tiles) if R else None,
-              plan.max_remote_tiles if R else 0, _lib.ptr(part_o), _lib.ptr(part_ml),
-              out.data_ptr(), lse.data_ptr(), _lib.stream_of(dev))
+              ptr["att_chunk"], ptr["self_tiles"], plan.n_self_tiles, at["sel"], R,
+              ptr["filtered"], plan.num_experts, at["tile_off"], at["row_off"], at["counts"],
+              at["rows"], at["tiles"], plan.max_remote_tiles if R else 0, work["part_o"],
+              work["part_ml"], out.data_ptr(), lse.data_ptr(), _lib.stream_of(dev))
     return out, lse
 
 
@@ -282,31 +338,23 @@ def backward(plan: PrefillPlan, q, k, v, out, lse, dout, rt: RouteResult | None)
     dev = q.device
     R = plan.remote
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    delta = torch.empty(2 * T * hq, dtype=torch.float32, device=dev)
-    part_dq = torch.empty((T * hq * R, d), dtype=q.dtype, device=dev) if R else None
+    buf = plan.bwd_work.alloc(dev)
+    work = plan.bwd_work.ptrs(buf)
+    at, ptr = rt.ptr if R else _NO_ROUTE, plan._ptrs
     args = [q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
             dout.data_ptr(), lse.data_ptr(), DTYPE_CODE[q.dtype], T, hq, plan.hkv, d,
-            d ** -0.5, plan.ptr("att_chunk"), plan.ptr("self_tiles"), plan.n_self_tiles,
-            plan.ptr("kv_tiles"), plan.n_kv_tiles,
-            _lib.ptr(rt.sel) if R else None, R, plan.ptr("filtered"), plan.num_experts,
-            _lib.ptr(rt.tile_off) if R else None, _lib.ptr(rt.row_off) if R else None,
-            _lib.ptr(rt.counts) if R else None, _lib.ptr(rt.rows) if R else None,
-            _lib.ptr(rt.tiles) if R else None,
-            plan.max_remote_tiles if R else 0, delta.data_ptr(), _lib.ptr(part_dq),
+            d ** -0.5, ptr["att_chunk"], ptr["self_tiles"], plan.n_self_tiles,
+            ptr["kv_tiles"], plan.n_kv_tiles, at["sel"], R, ptr["filtered"], plan.num_experts,
+            at["tile_off"], at["row_off"], at["counts"], at["rows"], at["tiles"],
+            plan.max_remote_tiles if R else 0, work["delta"], work["part_dq"],
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr()]
-    ks = plan.kv_splits
-    # row-split workspace: the device-built schedule, then fp32 partial slots
-    part_dkv = (torch.empty(_lib.load().moba_hip_prefill_bwd_work(plan.n_kv_tiles, ks, d),
-                            dtype=torch.uint8, device=dev) if ks > 1 else None)
-    # expert rows of q / dO / lse / delta packed contiguously for the key-major kernel
-    pack = (torch.empty(T * hq * R * (4 * d + 8), dtype=torch.uint8, device=dev)
-            if R and d <= 128 else None)
-    st = _lib.stream_of(dev)
-    _lib.call("moba_hip_prefill_bwd_tiles", *args, 1, ks, _lib.ptr(part_dkv), _lib.ptr(pack), st)
+    tail = (plan.kv_splits, work["part_dkv"], work["pack"], _lib.stream_of(dev))
     events = DKDV_EVENTS
-    if events is not None:
+    if events is None:
+        _lib.call("moba_hip_prefill_bwd_tiles", *args, 3, *tail)
+    else:
+        _lib.call("moba_hip_prefill_bwd_tiles", *args, 1, *tail)
         events[0].record()
-    _lib.call("moba_hip_prefill_bwd_tiles", *args, 2, ks, _lib.ptr(part_dkv), _lib.ptr(pack), st)
-    if events is not None:
+        _lib.call("moba_hip_prefill_bwd_tiles", *args, 2, *tail)
         events[1].record()
     return dq, dk, dv
