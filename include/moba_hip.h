@@ -122,14 +122,18 @@ int moba_hip_prefill_fwd(const void* q, const void* k, const void* v, int dtype,
                          void* out, float* lse, void* stream);
 
 /* The same with the tiles that moba_hip_prefill_route wrote: a remote
- * workgroup starts from its entry instead of a search of tile_off. */
+ * workgroup starts from its entry instead of a search of tile_off.  few_long
+ * (0 when unknown; any value gives the same results up to rounding): bit 0 when
+ * the longest self tile takes as long as the launch would if its work were
+ * spread evenly, bit 1 the same for the remote tiles. */
 int moba_hip_prefill_fwd_tiles(const void* q, const void* k, const void* v, int dtype, int T,
                                int Hq, int Hkv, int D, float scale, const int* cu_chunk,
                                const int* self_tiles, int n_self_tiles, const int* sel, int R,
                                const int* filtered, int E, const int* tile_off,
                                const int* row_off, const int* counts, const int* rows,
-                               const int* tiles, int max_remote_tiles, void* part_o,
-                               float* part_ml, void* out, float* lse, void* stream);
+                               const int* tiles, int max_remote_tiles, int few_long,
+                               void* part_o, float* part_ml, void* out, float* lse,
+                               void* stream);
 
 /* Backward of moba_hip_prefill_fwd with the GLOBAL O and LSE.
  * Replaces OptMixedAttention.backward (src/moba_opt/mixed_attention.py:141-225):

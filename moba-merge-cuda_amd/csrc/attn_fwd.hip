@@ -72,14 +72,17 @@ struct FwdArgs {
 // 3570 / 1425 -> 3415 / 1346; T 8192, 16/4 heads, D 256, chunk 1024 455 / 206
 // -> 289 / 171.  A fourth wave at 128 dims spills and is slower (3510 / 1460),
 // and so are 32 keys up to 64 dims (16/2 heads, T 16384: remote 264 -> 279).
+// A launch of few, long tiles (`few_long`) is bound by its longest tile instead,
+// where half the barriers per key count: 64 keys there up to 128 dims (full
+// causal attention over 3000 tokens, 8 heads, D 128: call 78 -> 62 us).
 template <int DP> constexpr int fwd_keys() { return DP <= 64 ? 64 : 32; }
-template <int DP> constexpr int fwd_waves() { return DP > 64 && DP <= 128 ? 3 : 2; }
+template <int DP, int KEYS> constexpr int fwd_waves() { return DP > 64 && DP <= 128 && KEYS == 32 ? 3 : 2; }
 constexpr float kRescaleSlack = 8.0f;  // log2 headroom before O is rescaled
 
-template <int DT, int DP, bool REMOTE, int QB>
-__global__ __launch_bounds__(256, fwd_waves<DP>()) void fwd_kernel(FwdArgs a) {
+template <int DT, int DP, bool REMOTE, int QB, int KEYS>
+__global__ __launch_bounds__(256, (fwd_waves<DP, KEYS>())) void fwd_kernel(FwdArgs a) {
   constexpr int NKS = DP / 16;  // k-steps of the QK^T contraction
-  constexpr int kBN = fwd_keys<DP>(), NKB = kBN / 32;  // keys per tile, 32-key blocks
+  constexpr int kBN = KEYS, NKB = kBN / 32;  // keys per tile, 32-key blocks
   constexpr int NDB = DP / 32;  // 32-row d blocks of O^T
   constexpr int TILE = kBN * DP;           // elements of one K or V tile
   constexpr int NB = DP / 8;                // 16-byte blocks per tile row
@@ -408,26 +411,42 @@ __global__ __launch_bounds__(256, fwd_waves<DP>()) void fwd_kernel(FwdArgs a) {
   }
 }
 
+template <int DT, int DP, bool REMOTE>
+void launch_one(const FwdArgs& a, int64_t wgs, bool few_long, hipStream_t st) {
+  const dim3 grid((unsigned)((wgs + 7) / 8 * 8));
+  constexpr int K = fwd_keys<DP>();
+  if constexpr (DP > 64 && DP <= 128) {
+    if (few_long) {
+      hipLaunchKernelGGL((fwd_kernel<DT, DP, REMOTE, attn_qb<DP>(), 64>), grid, dim3(256), 0, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((fwd_kernel<DT, DP, REMOTE, attn_qb<DP>(), K>), grid, dim3(256), 0, st, a);
+}
+
+// few_long: bit 0 for the self tiles, bit 1 for the remote ones (see
+// moba_hip_prefill_fwd_tiles).
 template <int DT, int DP>
-int launch_fwd(const FwdArgs& a, int n_self_tiles, int max_remote_tiles, hipStream_t st) {
+int launch_fwd(const FwdArgs& a, int n_self_tiles, int max_remote_tiles, int few_long,
+               hipStream_t st) {
   if (max_remote_tiles > 0 && a.R > 0) {
-    hipLaunchKernelGGL((fwd_kernel<DT, DP, true, attn_qb<DP>()>), dim3((max_remote_tiles + 7) / 8 * 8), dim3(256), 0, st, a);
+    launch_one<DT, DP, true>(a, max_remote_tiles, few_long & 2, st);
     int rc = moba_launch_status("prefill_fwd(remote)");
     if (rc) return rc;
   }
   if (n_self_tiles > 0) {
-    hipLaunchKernelGGL((fwd_kernel<DT, DP, false, attn_qb<DP>()>), dim3((unsigned)(((int64_t)n_self_tiles * a.G + 7) / 8 * 8)), dim3(256), 0, st, a);
+    launch_one<DT, DP, false>(a, (int64_t)n_self_tiles * a.G, few_long & 1, st);
     return moba_launch_status("prefill_fwd(self)");
   }
   return MOBA_OK;
 }
 
 template <int DT>
-int dispatch_fwd(const FwdArgs& a, int n_self, int max_remote, hipStream_t st) {
-  if (a.D <= 32) return launch_fwd<DT, 32>(a, n_self, max_remote, st);
-  if (a.D <= 64) return launch_fwd<DT, 64>(a, n_self, max_remote, st);
-  if (a.D <= 128) return launch_fwd<DT, 128>(a, n_self, max_remote, st);
-  return launch_fwd<DT, 256>(a, n_self, max_remote, st);
+int dispatch_fwd(const FwdArgs& a, int n_self, int max_remote, int few_long, hipStream_t st) {
+  if (a.D <= 32) return launch_fwd<DT, 32>(a, n_self, max_remote, few_long, st);
+  if (a.D <= 64) return launch_fwd<DT, 64>(a, n_self, max_remote, few_long, st);
+  if (a.D <= 128) return launch_fwd<DT, 128>(a, n_self, max_remote, few_long, st);
+  return launch_fwd<DT, 256>(a, n_self, max_remote, few_long, st);
 }
 
 }  // namespace
@@ -446,8 +465,9 @@ extern "C" int moba_hip_prefill_fwd_tiles(const void* q, const void* k, const vo
                                           int n_self_tiles, const int* sel, int R,
                                           const int* filtered, int E, const int* tile_off,
                                           const int* row_off, const int* counts, const int* rows,
-                                          const int* tiles, int max_remote_tiles, void* part_o,
-                                          float* part_ml, void* out, float* lse, void* stream) {
+                                          const int* tiles, int max_remote_tiles, int few_long,
+                                          void* part_o, float* part_ml, void* out, float* lse,
+                                          void* stream) {
   if (dtype != 0 && dtype != 1) { moba_set_error("prefill_fwd: dtype must be 0 (bf16) or 1 (fp16)"); return MOBA_ERR_ARG; }
   if (D < 8 || D > 256 || D % 8) { moba_set_error("prefill_fwd: head_dim must be a multiple of 8 in [8,256]"); return MOBA_ERR_ARG; }
   if (Hq < 1 || Hkv < 1 || Hq % Hkv) { moba_set_error("prefill_fwd: Hq must be a positive multiple of Hkv"); return MOBA_ERR_ARG; }
@@ -464,8 +484,8 @@ extern "C" int moba_hip_prefill_fwd_tiles(const void* q, const void* k, const vo
   a.part_o = (uint16_t*)part_o; a.part_ml = part_ml;
   a.out = (uint16_t*)out; a.lse = lse;
   hipStream_t st = (hipStream_t)stream;
-  return dtype == 0 ? dispatch_fwd<0>(a, n_self_tiles, R > 0 ? max_remote_tiles : 0, st)
-                    : dispatch_fwd<1>(a, n_self_tiles, R > 0 ? max_remote_tiles : 0, st);
+  return dtype == 0 ? dispatch_fwd<0>(a, n_self_tiles, R > 0 ? max_remote_tiles : 0, few_long, st)
+                    : dispatch_fwd<1>(a, n_self_tiles, R > 0 ? max_remote_tiles : 0, few_long, st);
 }
 
 extern "C" int moba_hip_prefill_fwd(const void* q, const void* k, const void* v, int dtype, int T,
@@ -477,6 +497,6 @@ extern "C" int moba_hip_prefill_fwd(const void* q, const void* k, const void* v,
                                     void* out, float* lse, void* stream) {
   return moba_hip_prefill_fwd_tiles(q, k, v, dtype, T, Hq, Hkv, D, scale, cu_chunk, self_tiles,
                                     n_self_tiles, sel, R, filtered, E, tile_off, row_off, counts,
-                                    rows, nullptr, max_remote_tiles, part_o, part_ml, out, lse,
+                                    rows, nullptr, max_remote_tiles, 0, part_o, part_ml, out, lse,
                                     stream);
 }

@@ -33,7 +33,7 @@ SIGNATURES = {
     "moba_hip_prefill_fwd": [_P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _P, _I, _P, _I, _P, _I,
                              _P, _P, _P, _P, _I, _P, _P, _P, _P, _P],
     "moba_hip_prefill_fwd_tiles": [_P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _P, _I, _P, _I, _P, _I,
-                                   _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P],
+                                   _P, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P],
     "moba_hip_prefill_bwd_tiles": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _P, _I, _P,
                                    _I, _P, _I, _P, _I, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P,
                                    _I, _I, _P, _P, _P],

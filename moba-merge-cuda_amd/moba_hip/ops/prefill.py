@@ -104,6 +104,14 @@ class PrefillPlan:
         rows_bound = cu[-1] * hq * self.remote
         max_tiles = min(max_tiles, -(-rows_bound // BLOCK_ROWS) + self.num_experts)
         self.max_remote_tiles = max_tiles
+        # launches bound by their longest tile: at least 1024 keys, and not less
+        # than an even share of all keys over the 768 workgroups (three per
+        # CU) that the chip holds
+        work = [min(r0 + BLOCK_ROWS, att_chunk[c + 1] - att_chunk[c])
+                for c, r0, _ in tiles if c >= 0]
+        self.few_long = int(bool(work) and max(work) >= 1024 and
+                            768 * max(work) >= sum(work) * self.groups)
+        self.few_long |= 2 * int(self.remote > 0 and chunk >= 1024 and max_tiles <= 768)
         self.chunk_start = [cu_chunk[c] for c in filtered]
         # key-major backward tiles: (chunk, first key, filtered index or -1)
         self.kv_block = dkdv_keys(head_dim)
@@ -322,8 +330,8 @@ def forward(plan: PrefillPlan, q, k, v, rt: RouteResult | None):
               DTYPE_CODE[q.dtype], T, hq, plan.hkv, d, d ** -0.5,
               ptr["att_chunk"], ptr["self_tiles"], plan.n_self_tiles, at["sel"], R,
               ptr["filtered"], plan.num_experts, at["tile_off"], at["row_off"], at["counts"],
-              at["rows"], at["tiles"], plan.max_remote_tiles if R else 0, work["part_o"],
-              work["part_ml"], out.data_ptr(), lse.data_ptr(), _lib.stream_of(dev))
+              at["rows"], at["tiles"], plan.max_remote_tiles if R else 0, plan.few_long,
+              work["part_o"], work["part_ml"], out.data_ptr(), lse.data_ptr(), _lib.stream_of(dev))
     return out, lse
 
 

@@ -483,7 +483,10 @@ def test_remote_tiles_given_or_searched(cuda_device, monkeypatch, hq, hkv, dim, 
     def searched(name, *args):
         if name in at:
             i = at[name]
-            args, name = args[:i] + args[i + 1:], name[:-len("_tiles")]
+            args = args[:i] + args[i + 1:]
+            if name == "moba_hip_prefill_fwd_tiles":   # its tile-length hint as well
+                args = args[:i + 1] + args[i + 2:]
+            name = name[:-len("_tiles")]
         call(name, *args)
     monkeypatch.setattr(P._lib, "call", searched)
     for a, b in zip(given, grads()):
@@ -511,3 +514,22 @@ def test_gate_bits_at_the_ends_of_the_range(cuda_device, dim, topk, scale):
     assert scale > 1 or ((tiny > 0) & (tiny < 2.0 ** -126)).any()
     if not nan.any():
         np.testing.assert_array_equal(rt.sel.cpu().numpy(), sel)
+
+
+@pytest.mark.parametrize("topk,hint", [(1, 1), (3, 3)])
+def test_few_long_tiles(cuda_device, topk, hint):
+    """Launches bound by their longest tile take 64-key tiles: the plan says so
+    for a long causal sequence and for long chunks, and the outputs match FP64
+    on the selected routes."""
+    T, chunk = 2300, 1100
+    q, k, v, cu, ml, g = prefill_inputs(2, 1, 128, (T,), torch.bfloat16, seed=37)
+    cfg = {"chunk_size": chunk, "topk": topk}
+    _, _, _, out, lse, plan = _run(q, k, v, cu, ml, cfg)
+    assert plan.few_long == hint
+    sel, att_chunk = None, cu.tolist()
+    if not plan.fallback:
+        sel, _, _, (att_chunk, _, _, _) = oracle_route(q, k, cu, chunk, topk)
+    o_ref, l_ref = O.attention_fwd(*(x.detach().double().cpu().numpy() for x in (q, k, v)),
+                                   att_chunk, sel)
+    assert_close_stats(out, o_ref, torch.bfloat16, "out")
+    np.testing.assert_allclose(lse.cpu().numpy(), l_ref, atol=2e-3, rtol=1e-4)
