@@ -533,3 +533,24 @@ def test_few_long_tiles(cuda_device, topk, hint):
                                    att_chunk, sel)
     assert_close_stats(out, o_ref, torch.bfloat16, "out")
     np.testing.assert_allclose(lse.cpu().numpy(), l_ref, atol=2e-3, rtol=1e-4)
+
+
+@pytest.mark.parametrize("hq,hkv,dim,lens,chunk,topk", [
+    (2, 1, 64, (129,), 64, 2),
+    (4, 2, 128, (700, 333), 96, 3),
+    (2, 1, 192, (515,), 128, 9),
+])
+def test_backward_in_one_call_or_two(cuda_device, monkeypatch, hq, hkv, dim, lens, chunk, topk):
+    """The row-split schedule built beside delta (both parts in one call) is the
+    one that the dK/dV call builds alone: the gradients are bitwise equal."""
+    from moba_hip.ops import prefill as P
+    q, k, v, cu, ml, g = prefill_inputs(hq, hkv, dim, lens, torch.bfloat16, seed=41)
+    _, _, _, out, lse, plan = _run(q, k, v, cu, ml, {"chunk_size": chunk, "topk": topk})
+    assert plan.kv_splits > 1, "the shape must take the row-split path"
+    rt = P.route(plan, q, k, 0) if plan.remote else None
+    out, lse = out.detach(), lse.detach()
+    one = P.backward(plan, q, k, v, out, lse, g, rt)
+    monkeypatch.setattr(P, "DKDV_EVENTS", [torch.cuda.Event() for _ in range(2)])
+    two = P.backward(plan, q, k, v, out, lse, g, rt)
+    for a, b in zip(one, two):
+        assert torch.equal(a, b)
