@@ -8,7 +8,7 @@
 // GQA gradients of the heads sharing a KV head are summed.
 //
 //   delta_kernel : Delta = rowsum(dO * O)                                  [T*Hq]
-//   dq_kernel<REMOTE> : query-major.  S^T = K Q^T, dP^T = V dO^T,
+//   dq_kernel<REMOTE> (dq2_kernel above 128 dims) : query-major.  S^T = K Q^T, dP^T = V dO^T,
 //        P = exp(S*scale - LSE), dS = P (dP - Delta), dQ^T += K^T dS^T.
 //        REMOTE tiles (expert rows) write dq partials into the row's slot;
 //        SELF tiles (causal within the chunk) add the slots in ascending order.
@@ -66,6 +66,57 @@ __global__ __launch_bounds__(256) void delta_kernel(const uint16_t* __restrict__
 }
 
 // --------------------------------------------------------------------- dq
+// Epilogue of one row.  Remote: dQ partial of the row's slot.  Self: the slots
+// are added in ascending order; one slot per iteration, its loads issued
+// together: slots below R are in the row's allocation, columns past D are
+// clamped (they reach only entries that are not stored), unselected slots
+// (sel < 0) add zero.
+template <int DT, int DP, bool REMOTE>
+__device__ __forceinline__ void finish_row(const BwdArgs& a, f32x16_t (&acc)[DP / 32], int64_t row,
+                                           int slot, int hh) {
+  constexpr int NDB = DP / 32;
+  const int D = a.D;
+  if constexpr (REMOTE) {
+    uint16_t* po = a.part_dq + (int64_t)slot * D;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) store_block<DT>(po, acc[db], a.scale, db, 8 * hh, D);
+  } else {
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[db][r] *= a.scale;
+    for (int jj = 0; jj < a.R; ++jj) {
+      const int64_t sl = row * a.R + jj;
+      const bool on = a.sel[sl] >= 0;
+      const uint16_t* po = a.part_dq + sl * D;
+      constexpr int NBL = NDB <= 4 ? NDB : 2;
+#pragma unroll
+      for (int d4 = 0; d4 < NDB; d4 += NBL) {
+        u16x8_t o[NBL][2];
+#pragma unroll
+        for (int db = 0; db < NBL; ++db)
+#pragma unroll
+          for (int m = 0; m < 2; ++m) {
+            const int d = (d4 + db) * 32 + 16 * m + 8 * hh;
+            o[db][m] = ld8(po + (d < D ? d : 0));
+          }
+#pragma unroll
+        for (int db = 0; db < NBL; ++db)
+#pragma unroll
+          for (int m = 0; m < 2; ++m) {
+            float x[8];
+            spread_piece<DT>(o[db][m], x);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[d4 + db][8 * m + i] += on ? x[i] : 0.0f;
+          }
+      }
+    }
+    uint16_t* orow = a.dq + row * D;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) store_block<DT>(orow, acc[db], 1.0f, db, 8 * hh, D);
+  }
+}
+
 // Per wave two blocks of 32 query rows; K/V tiles of 64 keys double-buffered
 // in LDS (row-major).  S^T = K Q^T and dP^T = V dO^T take K / V rows as the A
 // operand; dQ^T = K^T dS^T reads K^T with the transposed LDS read.
@@ -121,6 +172,7 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       h[qb] = kh * a.G + g;
+      slot[qb] = 0;
       s[qb] = s_wave0 + qb * 32 + qi;
       valid[qb] = s[qb] < c_end;
       if (!valid[qb]) s[qb] = k_hi - 1;
@@ -129,19 +181,13 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
   const int wave_s = __builtin_amdgcn_readfirstlane(wave);
   // Lane l of wave w loads blocks j = (n * 4 + w) * 64 + l: row j / NB,
   // physical block j % NB.  The row advances by 256 / NB per n, a multiple of
-  // 16 when DP <= 128, and the swizzle depends on the row mod 16 only, so
-  // every n has the same column and its offset is the n = 0 offset plus a
-  // uniform step (added per load, not held in NDMA registers).
-  constexpr bool UNI = (256 / NB) % 16 == 0;
-  uint32_t voff[UNI ? 1 : NDMA];
-  bool vok[UNI ? 1 : NDMA];
-#pragma unroll
-  for (int n = 0; n < (UNI ? 1 : NDMA); ++n) {
-    const int j = (n * 4 + wave_s) * 64 + lane, row = j / NB;
-    const int col = swz<DP>(row, (j % NB) * 8) - row * DP;  // swizzle is an involution
-    voff[n] = (uint32_t)(((row * a.Hkv + kh) * D + col) * 2);
-    vok[n] = col < D;
-  }
+  // 16, and the swizzle depends on the row mod 16 only, so every n has the
+  // same column and its offset is the n = 0 offset plus a uniform step (added
+  // per load, not held in NDMA registers).
+  static_assert((256 / NB) % 16 == 0, "head dims up to 128");
+  const int vj = wave_s * 64 + lane, vrow = vj / NB;
+  const int vcol = swz<DP>(vrow, (vj % NB) * 8) - vrow * DP;  // swizzle is an involution
+  const uint32_t voff = (uint32_t)(((vrow * a.Hkv + kh) * D + vcol) * 2);
   const uint32_t vstep = (uint32_t)((256 / NB) * a.Hkv * D * 2);
   const int n_keys = k_hi - k_lo;
   const uint32_t nrec = (uint32_t)((((int64_t)(n_keys - 1) * a.Hkv + kh + 1) * D) * 2);
@@ -150,11 +196,11 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
   const uint32_t tile_bytes = (uint32_t)(kBN * a.Hkv * D * 2);
   auto dma = [&](uint16_t* Kd, uint16_t* Vd, int it) {
     const uint32_t soff = (uint32_t)it * tile_bytes;
-    const uint32_t v0 = opaque(voff[0]);
+    const uint32_t v0 = opaque(voff);
 #pragma unroll
     for (int n = 0; n < NDMA; ++n) {
-      if (vok[UNI ? 0 : n]) {
-        const uint32_t vo = UNI ? v0 + n * vstep : voff[n];
+      if (vcol < D) {
+        const uint32_t vo = v0 + n * vstep;
         load_lds16(make_rsrc(kbase, nrec), Kd + (n * 4 + wave_s) * 64 * 8, vo, soff);
         load_lds16(make_rsrc(vbase, nrec), Vd + (n * 4 + wave_s) * 64 * 8, vo, soff);
       }
@@ -170,12 +216,9 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
     __syncthreads();
   }
   // The first K / V tile goes out before the query rows: an expert's rows
-  // wait for their row list, the tile only for the workgroup's entry (above
-  // 128 dims the rows come first and each load is guarded: otherwise the
-  // kernel spills 325 registers).  Rows past the tile's end load the last
-  // row's data and are never written.
-  constexpr bool TILE_FIRST = DP <= 128;
-  if constexpr (TILE_FIRST) dma(K0, V0, 0);
+  // wait for their row list, the tile only for the workgroup's entry.  Rows
+  // past the tile's end load the last row's data and are never written.
+  dma(K0, V0, 0);
   u16x8_t qf[QB][NKS], gf[QB][NKS];
   float lse2[QB], lk[QB], dl[QB];
 #pragma unroll
@@ -190,21 +233,16 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
       const int d = ks * 16 + hh * 8, dc = d < D ? d : 0;
-      if constexpr (TILE_FIRST) {
-        const u16x8_t xq = ld8(a.q + row * D + dc), xg = ld8(a.dout + row * D + dc);
-        qf[qb][ks] = d < D ? xq : zero8();
-        gf[qb][ks] = d < D ? xg : zero8();
-      } else {
-        qf[qb][ks] = valid[qb] && d < D ? ld8(a.q + row * D + d) : zero8();
-        gf[qb][ks] = valid[qb] && d < D ? ld8(a.dout + row * D + d) : zero8();
-      }
+      const u16x8_t xq = ld8(a.q + row * D + dc), xg = ld8(a.dout + row * D + dc);
+      qf[qb][ks] = d < D ? xq : zero8();
+      gf[qb][ks] = d < D ? xg : zero8();
     }
     const float lr = a.lse[row];
     lse2[qb] = lr * kLog2e;
     lk[qb] = lr / a.scale;
     dl[qb] = a.delta[row];
   }
-  if constexpr (REMOTE && DP <= 128) {
+  if constexpr (REMOTE) {
     // The key-major dK/dV kernel reads the expert rows packed contiguously in
     // row_off order; this kernel holds exactly those rows, so it writes the
     // packed q / dO / lse_k / delta (the values delta_kernel and the loads above
@@ -228,7 +266,6 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
     }
   }
 
-  if constexpr (!TILE_FIRST) dma(K0, V0, 0);
   const uint32_t kbase0 = swz_b128_base<DP>(lane);
   const uint32_t trb0 = swz_tr_base<DP>(lane, 0), trb1 = swz_tr_base<DP>(lane, 1);
 
@@ -385,52 +422,209 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
   }
 
 #pragma unroll
-  for (int qb = 0; qb < QB; ++qb) {
-    if (!valid[qb]) continue;
-    const int64_t row = (int64_t)s[qb] * a.Hq + h[qb];
-    if constexpr (REMOTE) {
-      uint16_t* po = a.part_dq + (int64_t)slot[qb] * D;
+  for (int qb = 0; qb < QB; ++qb)
+    if (valid[qb])
+      finish_row<DT, DP, REMOTE>(a, acc[qb], (int64_t)s[qb] * a.Hq + h[qb], slot[qb], hh);
+}
+
+// --------------------------------------------- dq, head dims 129..256
+// The same work and tiles of 128 rows, by 4 wave pairs of 32 rows.  Here Q, dO
+// and dQ of 32 rows take 256 registers: one wave that holds all three has them
+// in both register files and moves operands between these for most MFMAs, alone
+// on its SIMD.  So a pair shares a SIMD and splits the products, over blocks of
+// 32 keys.  At step t:
+//   role S (Q, dO):  S^T = K_t Q^T, dP^T = V_t dO^T, dS_t to LDS (the operand
+//                    as its lane holds it: 2 KB per pair)
+//   role G (dQ):     dQ^T += K_{t-1}^T dS_{t-1}
+// Role S goes first (s_setprio): role G's MFMAs run under its element-wise
+// work.  K has 4 stages and V 3 (t - 1, t, and two blocks of loads in flight);
+// one barrier a step.  The sums are those of dq_kernel, in its order.
+// T 8192, 16/4 heads, chunk 1024, top-3, D 256: remote 570 -> 425-454 us, self
+// 188 -> 195-205 us, the training step 1780 -> 1681 us; matrix units busy 44%
+// and 28% of the CU cycles, LDS 25% and 16% with no bank conflicts.  2 to 5
+// (role S) or 4 to 8 (role G) operand reads in flight and no priority measure
+// the same, role G first 8% slower; the element-wise work of block t - 1 between
+// role S's MFMAs of block t (two S^T and dP^T in registers, five K stages) is
+// 2% slower.
+constexpr int kBK = 32;  // keys per block
+
+template <int DT, int DP, bool REMOTE>
+__global__ __launch_bounds__(512, 2) void dq2_kernel(BwdArgs a) {
+  constexpr int NKS = DP / 16, NDB = DP / 32, NB = DP / 8;
+  constexpr int TILE = kBK * DP, NDMA = kBK * NB / 512;
+  constexpr int NSK = 4, NSV = 3;
+  __shared__ __attribute__((aligned(16))) uint16_t Ks[NSK * TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t Vs[NSV * TILE];
+  __shared__ __attribute__((aligned(16))) u16x8_t Ds[2][4][2][64];  // dS of block & 1, per pair
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int pair = wave & 3, qi = lane & 31, hh = lane >> 5;
+  const int D = a.D;
+  int s, h, slot = 0, kh, k_lo, k_hi, s_wave0 = 0;
+  bool valid;
+  if constexpr (REMOTE) {
+    const ExpertTile x = expert_tile<128>(a);
+    if (x.rows == 0) return;
+    kh = x.kh;
+    k_lo = x.k_lo;
+    k_hi = x.k_hi;
+    const int local = pair * 32 + qi;
+    valid = local < x.rows;
+    const int packed = a.rows[x.row0 + min(local, x.rows - 1)];  // (row << 3) | j
+    slot = (packed >> 3) * a.R + (packed & 7);
+    s = (packed >> 3) / a.Hq;
+    h = (packed >> 3) % a.Hq;
+  } else {
+    const int t = xcd_contiguous(blockIdx.x, a.n_self_wg);
+    if (t < 0) return;
+    const int e = t / a.G, g = t - e * a.G;
+    const int c = a.self_tiles[3 * e];
+    if (c < 0) return;
+    const int row0 = a.self_tiles[3 * e + 1];
+    kh = a.self_tiles[3 * e + 2];
+    k_lo = a.cu_chunk[c];
+    const int c_end = a.cu_chunk[c + 1];
+    k_hi = min(c_end, k_lo + row0 + 128);
+    s_wave0 = k_lo + row0 + pair * 32;
+    h = kh * a.G + g;
+    s = s_wave0 + qi;
+    valid = s < c_end;
+    if (!valid) s = k_hi - 1;
+  }
+  const int64_t row = (int64_t)s * a.Hq + h;
+
+  // Thread t loads 16-byte blocks n * 512 + t of a tile.  Columns past D and
+  // keys past the end read past num_records, i.e. zeros; a block past the last
+  // loads zeros into a stage nobody reads, so every block is 2 * NDMA loads.
+  const int n_keys = k_hi - k_lo, nblk = (n_keys + kBK - 1) / kBK;
+  const uint32_t nrec = (uint32_t)((((int64_t)(n_keys - 1) * a.Hkv + kh + 1) * D) * 2);
+  const __amdgpu_buffer_rsrc_t rk = make_rsrc(a.k + (int64_t)k_lo * a.Hkv * D, nrec);
+  const __amdgpu_buffer_rsrc_t rv = make_rsrc(a.v + (int64_t)k_lo * a.Hkv * D, nrec);
+  auto dma = [&](int t, int sk, int sv) __attribute__((always_inline)) {
+    const int tid = (int)opaque(threadIdx.x);
 #pragma unroll
-      for (int db = 0; db < NDB; ++db) store_block<DT>(po, acc[qb][db], a.scale, db, 8 * hh, D);
-    } else {
+    for (int n = 0; n < NDMA; ++n) {
+      const int j = n * 512 + tid, r = j / NB, col = swz<DP>(r, (j % NB) * 8) - r * DP;
+      const int key = t * kBK + r;
+      const uint32_t off = (key < n_keys && col < D) ? (uint32_t)((key * a.Hkv + kh) * D + col) * 2 : nrec;
+      const int jb = (n * 512 + wave * 64) * 8;
+      dma_lds16(rk, Ks + sk * TILE + jb, off, 0);
+      dma_lds16(rv, Vs + sv * TILE + jb, off, 0);
+    }
+  };
+  // causal blocks wholly above the pair's rows add exact zeros
+  auto skipped = [&](int t) __attribute__((always_inline)) {
+    return t < 0 || t >= nblk || (!REMOTE && k_lo + t * kBK > s_wave0 + 31);
+  };
+  dma(0, 0, 0);
+  dma(1, 1, 1);
+
+  // One step per block and one more, so that role G finishes the last.  Loads
+  // run two blocks ahead; at the step's end those of the next block have landed.
+  auto steps = [&](auto&& work) __attribute__((always_inline)) {
+    lds_barrier();
+    int sv = 0;
+    for (int t = 0; t <= nblk; ++t) {
+      dma(t + 2, (t + 2) % NSK, sv == 0 ? 2 : sv - 1);
+      __builtin_amdgcn_sched_barrier(0);
+      work(t, sv);
+      sv = sv == NSV - 1 ? 0 : sv + 1;
+      wait_vmcnt<2 * NDMA>();
+      lds_barrier();
+    }
+    wait_vmcnt<0>();  // no load may reach the LDS of the next workgroup
+  };
+
+  if (wave < 4) {
+    u16x8_t qf[NKS], gf[NKS];
 #pragma unroll
-      for (int db = 0; db < NDB; ++db)
+    for (int ks = 0; ks < NKS; ++ks) {
+      const int d = ks * 16 + hh * 8, dc = d < D ? d : 0;
+      const u16x8_t xq = ld8(a.q + row * D + dc), xg = ld8(a.dout + row * D + dc);
+      qf[ks] = d < D ? xq : zero8();
+      gf[ks] = d < D ? xg : zero8();
+    }
+    const float nl = -a.lse[row] * kLog2e, dl = a.delta[row], c2 = a.scale_log2;
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // rows and the first two blocks landed
+    const uint32_t kq0 = swz_b128_base<DP>(lane);
+    __builtin_amdgcn_s_setprio(1);
+    steps([&](int t, int sv) __attribute__((always_inline)) {
+      if (skipped(t)) return;
+      const uint16_t* Kb = Ks + (t % NSK) * TILE;
+      const uint16_t* Vb = Vs + sv * TILE;
+      const uint32_t kq = opaque(kq0);
+      f32x16_t sa = zero16(), pa = zero16();
+      constexpr int PF = 3;  // operand reads ahead of their MFMAs
+      u16x8_t ka[PF], va[PF];
+      auto rd = [&](int i) __attribute__((always_inline)) {
+        const uint32_t o = swz_b128<DP>(kq, i);
+        ka[i % PF] = lds8(Kb, o);
+        va[i % PF] = lds8(Vb, o);
+      };
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[qb][db][r] *= a.scale;
-      // one slot per iteration, its loads issued together: slots below R are
-      // in the row's allocation, columns past D are clamped (they reach only
-      // entries that are not stored), unselected slots (sel < 0) add zero
-      for (int jj = 0; jj < a.R; ++jj) {
-        const int64_t sl = row * a.R + jj;
-        const bool on = a.sel[sl] >= 0;
-        const uint16_t* po = a.part_dq + sl * D;
-        constexpr int NBL = NDB <= 4 ? NDB : 2;
+      for (int i = 0; i < PF; ++i) rd(i);
 #pragma unroll
-        for (int d4 = 0; d4 < NDB; d4 += NBL) {
-          u16x8_t o[NBL][2];
+      for (int ks = 0; ks < NKS; ++ks) {
+        const u16x8_t xk = ka[ks % PF], xv = va[ks % PF];
+        if (ks + PF < NKS) rd(ks + PF);
+        sa = mfma32<DT>(xk, qf[ks], sa);
+        pa = mfma32<DT>(xv, gf[ks], pa);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      float p[16];
 #pragma unroll
-          for (int db = 0; db < NBL; ++db)
+      for (int r = 0; r < 16; ++r) p[r] = fast_exp2(fmaf(sa[r], c2, nl));
+      const int kt0 = k_lo + t * kBK;
+      if (kt0 + kBK > k_hi || (!REMOTE && kt0 + kBK - 1 > s_wave0)) {
 #pragma unroll
-            for (int m = 0; m < 2; ++m) {
-              const int d = (d4 + db) * 32 + 16 * m + 8 * hh;
-              o[db][m] = ld8(po + (d < D ? d : 0));
-            }
-#pragma unroll
-          for (int db = 0; db < NBL; ++db)
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-              float x[8];
-              spread_piece<DT>(o[db][m], x);
-#pragma unroll
-              for (int i = 0; i < 8; ++i) acc[qb][d4 + db][8 * m + i] += on ? x[i] : 0.0f;
-            }
+        for (int r = 0; r < 16; ++r) {
+          const int key = kt0 + 8 * (r >> 2) + 4 * hh + (r & 3);
+          p[r] = (key < k_hi && (REMOTE || key <= s)) ? p[r] : 0.0f;
         }
       }
-      uint16_t* orow = a.dq + row * D;
 #pragma unroll
-      for (int db = 0; db < NDB; ++db) store_block<DT>(orow, acc[qb][db], 1.0f, db, 8 * hh, D);
-    }
+      for (int r = 0; r < 16; ++r) p[r] *= pa[r] - dl;
+      Ds[t & 1][pair][0][lane] = pack8<DT>(p);
+      Ds[t & 1][pair][1][lane] = pack8<DT>(p + 8);
+    });
+  } else {
+    f32x16_t acc[NDB];
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) acc[db] = zero16();
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    const uint32_t trb0 = swz_tr_base<DP>(lane, 0), trb1 = swz_tr_base<DP>(lane, 1);
+    steps([&](int t, int) __attribute__((always_inline)) {
+      if (skipped(t - 1)) return;
+      const uint16_t* Kb = Ks + ((t - 1) % NSK) * TILE;
+      const uint32_t t0 = opaque(trb0), t1 = opaque(trb1);
+      const u16x8_t ds[2] = {Ds[(t - 1) & 1][pair][0][lane], Ds[(t - 1) & 1][pair][1][lane]};
+      constexpr int N2 = 2 * NDB, PF = 4;  // step i: d block i / 2, 16-key half i % 2
+      u16x8_t ring[PF];
+      auto rd = [&](int i) __attribute__((always_inline)) {
+        const uint32_t ro = (i % 2) * 16 * DP * 2;
+        return lds_tr8(Kb, ro + swz_tr<DP>(t0, i / 2), ro + swz_tr<DP>(t1, i / 2));
+      };
+#pragma unroll
+      for (int i = 0; i < PF; ++i) ring[i] = rd(i);
+#pragma unroll
+      for (int i = 0; i < N2; ++i) {
+        const u16x8_t kt = ring[i % PF];
+        if (i + PF < N2) ring[i % PF] = rd(i + PF);
+        acc[i / 2] = mfma32<DT>(kt, ds[i % 2], acc[i / 2]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+    if (valid) finish_row<DT, DP, REMOTE>(a, acc, row, slot, hh);
   }
+}
+
+template <int DT, int DP, bool REMOTE>
+void launch_dq(const BwdArgs& a, unsigned grid, hipStream_t st) {
+  if constexpr (DP <= 128)
+    hipLaunchKernelGGL((dq_kernel<DT, DP, REMOTE, attn_qb<DP>()>), dim3(grid), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((dq2_kernel<DT, DP, REMOTE>), dim3(grid), dim3(512), 0, st, a);
 }
 
 // Row-split schedule of the key-major kernels, built on the device because
@@ -641,9 +835,9 @@ int launch_bwd(const BwdArgs& a, int n_self, int n_kv, int max_remote, int parts
       hipLaunchKernelGGL(delta_kernel<DT>, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0,
                          st, a.out, a.dout, a.lse, rows, a.D, a.delta, a.scale, a.lse_k);
     if (max_remote > 0 && a.R > 0)
-      hipLaunchKernelGGL((dq_kernel<DT, DP, true, attn_qb<DP>()>), dim3((max_remote + 7) / 8 * 8), dim3(256), 0, st, a);
+      launch_dq<DT, DP, true>(a, (unsigned)((max_remote + 7) / 8 * 8), st);
     if (n_self > 0)
-      hipLaunchKernelGGL((dq_kernel<DT, DP, false, attn_qb<DP>()>), dim3((unsigned)(((int64_t)n_self * a.G + 7) / 8 * 8)), dim3(256), 0, st, a);
+      launch_dq<DT, DP, false>(a, (unsigned)(((int64_t)n_self * a.G + 7) / 8 * 8), st);
   }
   if ((parts & 2) && n_kv > 0) {
     // kKvTileKeys keys per workgroup in every kernel; the host's key tiles match

@@ -42,12 +42,6 @@ namespace {
 constexpr int kWaveKeys = 32;   // keys per wave
 constexpr int kStages = 3;      // LDS stages of (Q, dO) tiles
 
-// s_waitcnt vmcnt(N), other counters untouched (N < 16).
-template <int N> MOBA_DEV void wait_vmcnt() {
-  static_assert(N >= 0 && N < 16, "vmcnt immediate");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | N);
-}
-
 template <int DT, int DP>
 __global__ __launch_bounds__(256, 2) void dkdv1_kernel(BwdArgs a) {
   constexpr int kRows = kv_rows<DP>();

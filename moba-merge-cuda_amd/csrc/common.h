@@ -277,6 +277,12 @@ MOBA_DEV void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// s_waitcnt vmcnt(N), other counters untouched (N < 16).
+template <int N> MOBA_DEV void wait_vmcnt() {
+  static_assert(N >= 0 && N < 16, "vmcnt immediate");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | N);
+}
+
 // Rows of a transposed accumulator (D layout: lane l holds column l % 32,
 // entries 8j + 4(l/32) + i of each 32-entry block) as 16-byte pieces: lanes l
 // and l + 32 exchange halves (v_permlane32_swap), after which lane l holds

@@ -554,3 +554,23 @@ def test_backward_in_one_call_or_two(cuda_device, monkeypatch, hq, hkv, dim, len
     two = P.backward(plan, q, k, v, out, lse, g, rt)
     for a, b in zip(one, two):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("hq,hkv,dim,lens,chunk,topk", [
+    (2, 2, 136, (1, 31, 33), 16, 3),     # single blocks, fewer rows than a pair
+    (4, 1, 256, (130, 257), 96, 3),      # partial last block, chunk end inside a pair's rows
+    (2, 1, 200, (700,), 200, 9),         # columns past D, several experts per row
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dq_edges_above_128_dims(cuda_device, dtype, hq, hkv, dim, lens, chunk, topk):
+    """The wave pairs of the wide dQ at the edges of blocks and rows, against FP64."""
+    q, k, v, cu, ml, g = prefill_inputs(hq, hkv, dim, lens, dtype, seed=43)
+    qr, kr, vr, out, lse, plan = _run(q, k, v, cu, ml, {"chunk_size": chunk, "topk": topk})
+    out.backward(g)
+    sel, att_chunk = None, cu.tolist()
+    if not plan.fallback:
+        sel, _, _, (att_chunk, _, _, _) = oracle_route(q, k, cu, chunk, topk)
+    qd, kd, vd, gd = (x.detach().double().cpu().numpy() for x in (q, k, v, g))
+    _, l_ref = O.attention_fwd(qd, kd, vd, att_chunk, sel)
+    dq_ref, _, _ = O.attention_bwd(qd, kd, vd, gd, att_chunk, sel, l_ref)
+    assert_grad_close(qr.grad, dq_ref, dtype, "dq")
