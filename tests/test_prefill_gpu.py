@@ -574,3 +574,42 @@ def test_dq_edges_above_128_dims(cuda_device, dtype, hq, hkv, dim, lens, chunk, 
     _, l_ref = O.attention_fwd(qd, kd, vd, att_chunk, sel)
     dq_ref, _, _ = O.attention_bwd(qd, kd, vd, gd, att_chunk, sel, l_ref)
     assert_grad_close(qr.grad, dq_ref, dtype, "dq")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dim", [64, 72, 128, 256])
+@pytest.mark.parametrize("remote", [False, True])
+def test_largest_weight_is_not_rounded(cuda_device, dtype, dim, remote):
+    """A row whose largest score lies among its first 64 keys, above the largest of
+    the first 32 by less than the rescale slack: its weight is 1 in the 16-bit
+    P whatever the key tile.  Beside it one weight of at most 2^-6.1 and nothing
+    else, so the output's error is its own rounding (half an ulp; a remote
+    partial is rounded so, too, and merging it alone gives it back), the second
+    weight's (2^-6.1 of an ulp at most, V lying in [1, 2)) and that of fp32."""
+    C = 64
+    gen = torch.Generator().manual_seed(47)
+    q, k, v = torch.zeros(2 * C, 1, dim), torch.zeros(2 * C, 1, dim), torch.zeros(2 * C, 1, dim)
+    big, other = 41, 3
+    rows = torch.arange(C, 2 * C) if remote else torch.arange(big, C)
+    # log2 gaps of 6.2 to 7.9 between the two keys, all else 2^-30 below
+    gap = 6.2 + 1.7 * torch.rand(len(rows), generator=gen)
+    k[:, 0, 0], k[:, 0, 1] = -64.0, 0.0
+    k[other, 0, 0], k[big, 0, 0], k[big, 0, 1] = 0.0, 0.0, 8.0
+    unit = np.log(2.0) * dim ** 0.5
+    q[rows, 0, 0] = float(unit)
+    q[rows, 0, 1] = gap * float(unit) / 8
+    v[:C] = 1.0 + torch.rand(C, 1, dim, generator=gen)
+    q, k, v = (x.to("cuda", dtype) for x in (q, k, v))
+    cu = torch.tensor([0, 2 * C] if remote else [0, C, 2 * C], device="cuda", dtype=torch.int32)
+    cfg = {"chunk_size": C, "topk": 2 if remote else 1}
+    _, _, _, out, _, plan = _run(q, k, v, cu, 2 * C if remote else C, cfg)
+    assert plan.remote == int(remote) and plan.few_long == 0
+    qd, kd, vd = (x.double().cpu().numpy()[:, 0] for x in (q, k, v))
+    r = rows.numpy()
+    s = qd[r] @ kd[:C].T * dim ** -0.5
+    s = np.where(remote | (np.arange(C)[None] <= r[:, None]), s, -np.inf)
+    p = np.exp(s - s.max(1, keepdims=True))
+    ref = p @ vd[:C] / p.sum(1, keepdims=True)
+    ulp = np.exp2(np.floor(np.log2(ref)) - (7 if dtype == torch.bfloat16 else 10))
+    err = np.abs(out.detach().double().cpu().numpy()[r, 0] - ref) / ulp
+    assert err.max() <= 0.5 + 2.0 ** -6 + 2.0 ** -7
