@@ -124,8 +124,8 @@ int moba_hip_prefill_fwd(const void* q, const void* k, const void* v, int dtype,
 /* The same with the tiles that moba_hip_prefill_route wrote: a remote
  * workgroup starts from its entry instead of a search of tile_off.  few_long
  * (0 when unknown; any value gives the same results up to rounding): bit 0 when
- * the longest self tile takes as long as the launch would if its work were
- * spread evenly, bit 1 the same for the remote tiles. */
+ * the longest self tile decides how long the launch takes, bit 1 the same for
+ * the remote tiles. */
 int moba_hip_prefill_fwd_tiles(const void* q, const void* k, const void* v, int dtype, int T,
                                int Hq, int Hkv, int D, float scale, const int* cu_chunk,
                                const int* self_tiles, int n_self_tiles, const int* sel, int R,

@@ -72,11 +72,16 @@ struct FwdArgs {
 // 3570 / 1425 -> 3415 / 1346; T 8192, 16/4 heads, D 256, chunk 1024 455 / 206
 // -> 289 / 171.  A fourth wave at 128 dims spills and is slower (3510 / 1460),
 // and so are 32 keys up to 64 dims (16/2 heads, T 16384: remote 264 -> 279).
-// A launch of few, long tiles (`few_long`) is bound by its longest tile instead,
-// where half the barriers per key count: 64 keys there up to 128 dims (full
-// causal attention over 3000 tokens, 8 heads, D 128: call 78 -> 62 us).
+// A launch that is bound by its longest tile (`few_long`) gains more from half
+// the barriers per key: 64 keys there, the 256-wide self kernel with one wave
+// per SIMD.  Full causal attention, 8 heads, 32 -> 64 keys, us: D 128, 512
+// tokens 18.0 -> 15.8, 3000 76 -> 62; D 192, 1024 tokens 51.9 -> 49.9, 6000
+// 271 -> 253.  The wide remote kernel has no such launches (4096 tokens, chunk
+// 1024, D 192, 2 heads 106.2 -> 106.5, 16/4 heads 176 -> 207).
 template <int DP> constexpr int fwd_keys() { return DP <= 64 ? 64 : 32; }
-template <int DP, int KEYS> constexpr int fwd_waves() { return DP > 64 && DP <= 128 && KEYS == 32 ? 3 : 2; }
+template <int DP, int KEYS> constexpr int fwd_waves() {
+  return DP > 128 && KEYS == 64 ? 1 : DP > 64 && DP <= 128 && KEYS == 32 ? 3 : 2;
+}
 constexpr float kRescaleSlack = 8.0f;  // log2 headroom before O is rescaled
 
 template <int DT, int DP, bool REMOTE, int QB, int KEYS>
@@ -422,7 +427,7 @@ template <int DT, int DP, bool REMOTE>
 void launch_one(const FwdArgs& a, int64_t wgs, bool few_long, hipStream_t st) {
   const dim3 grid((unsigned)((wgs + 7) / 8 * 8));
   constexpr int K = fwd_keys<DP>();
-  if constexpr (DP > 64 && DP <= 128) {
+  if constexpr (DP > 64 && (DP <= 128 || !REMOTE)) {
     if (few_long) {
       hipLaunchKernelGGL((fwd_kernel<DT, DP, REMOTE, attn_qb<DP>(), 64>), grid, dim3(256), 0, st, a);
       return;

@@ -229,3 +229,25 @@ def test_plan_cache_is_thread_safe():
     for t in threads:
         t.join()
     assert not errors, errors[:3]
+
+
+@pytest.mark.parametrize("lens,hq,hkv,dim,chunk,topk,hint", [
+    # one side and the other of each line of the rule, at measured launches
+    ((512,), 8, 8, 128, 512, 1, 1), ((128,) * 64, 8, 8, 128, 512, 1, 0),
+    ((256,) * 36, 8, 8, 128, 512, 1, 0), ((1024,) * 9, 8, 8, 96, 512, 1, 1),
+    ((1024,) * 12, 8, 8, 128, 512, 1, 0), ((2048,) * 6, 8, 8, 128, 512, 1, 1),
+    ((4096,) * 3, 8, 8, 128, 512, 1, 1), ((4096,) * 4, 8, 8, 128, 512, 1, 0),
+    ((8192,), 16, 16, 128, 512, 1, 1), ((12000,) + (300,) * 100, 4, 4, 128, 512, 1, 1),
+    ((6000,), 8, 8, 192, 512, 1, 1), ((2048,) * 3, 8, 8, 136, 512, 1, 1),
+    ((2048,) * 4, 8, 8, 136, 512, 1, 0), ((16384,), 4, 4, 256, 512, 1, 0),
+    # remote tiles: 384, 672 and 398 of them, short chunks, wide heads
+    ((4096,), 8, 8, 128, 1024, 3, 3), ((4096,), 14, 14, 128, 1024, 3, 1),
+    ((2048,), 12, 2, 128, 256, 3, 3), ((1024,), 4, 2, 128, 64, 3, 0),
+    ((4096,), 2, 2, 192, 1024, 3, 1), ((4096,), 16, 4, 192, 1024, 3, 0),
+])
+def test_long_tile_hint(lens, hq, hkv, dim, chunk, topk, hint):
+    from itertools import accumulate
+    from moba_hip.ops.prefill import PrefillPlan
+    plan = PrefillPlan([0, *accumulate(lens)], chunk, hq, hkv, dim, topk, "cpu",
+                       fallback=topk == 1)
+    assert plan.few_long == hint

@@ -613,3 +613,25 @@ def test_largest_weight_is_not_rounded(cuda_device, dtype, dim, remote):
     ulp = np.exp2(np.floor(np.log2(ref)) - (7 if dtype == torch.bfloat16 else 10))
     err = np.abs(out.detach().double().cpu().numpy()[r, 0] - ref) / ulp
     assert err.max() <= 0.5 + 2.0 ** -6 + 2.0 ** -7
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dim", [72, 96, 120, 128, 136, 192, 256])
+@pytest.mark.parametrize("topk,lens,chunk", [
+    (1, (515, 33, 300), 512),     # partial 32- and 64-key tiles, sequences below one tile
+    (3, (1033, 70, 290), 260),    # a chunk end inside a tile, a last chunk below a tile
+])
+def test_64_key_tiles(cuda_device, dtype, dim, topk, lens, chunk):
+    """The kernels of long tiles over dtypes and head dims (columns past D in
+    both widths) and sequences that end inside a tile, against FP64 on the
+    selected routes."""
+    q, k, v, cu, ml, _ = prefill_inputs(4, 2, dim, lens, dtype, seed=53)
+    _, _, _, out, lse, plan = _run(q, k, v, cu, ml, {"chunk_size": chunk, "topk": topk})
+    assert plan.few_long == (1 if topk == 1 or dim > 128 else 3)
+    sel, att_chunk = None, cu.tolist()
+    if not plan.fallback:
+        sel, _, _, (att_chunk, _, _, _) = oracle_route(q, k, cu, chunk, topk)
+    o_ref, l_ref = O.attention_fwd(*(x.detach().double().cpu().numpy() for x in (q, k, v)),
+                                   att_chunk, sel)
+    assert_close_stats(out, o_ref, dtype, "out")
+    np.testing.assert_allclose(lse.cpu().numpy(), l_ref, atol=2e-3, rtol=1e-4)
