@@ -277,6 +277,15 @@ MOBA_DEV void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Orders a wave's LDS accesses around it: what its lanes wrote before, all its
+// lanes read after.  The LDS serves a wave's accesses in order, so this costs no
+// instruction; it keeps the compiler from moving them across.
+MOBA_DEV void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // s_waitcnt vmcnt(N), other counters untouched (N < 16).
 template <int N> MOBA_DEV void wait_vmcnt() {
   static_assert(N >= 0 && N < 16, "vmcnt immediate");

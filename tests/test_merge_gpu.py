@@ -143,3 +143,43 @@ def test_merge_keeps_the_first_kmax_partials(cuda_device, kmax, counts, dtype):
     np.testing.assert_allclose(lse.double().cpu().numpy(), ref[1], atol=2e-6, rtol=1e-6)
     with pytest.raises(RuntimeError, match="capacity exceeded"):
         merge_forward(so, sl, ro, rl, mp, kmax=kmax)
+
+
+@pytest.mark.parametrize("kmax", [1, 2, 8])
+@pytest.mark.parametrize("rows", ["one", "two in turn", "sixteen in turn", "runs of ten",
+                                  "one among many"])
+def test_merge_of_crowded_rows(cuda_device, rows, kmax):
+    """Mappings in which waves meet in a few rows: the first kmax partials of
+    each row are merged, and the call takes no more than ten times one whose
+    partials are spread out (minima on one address are served one by one: 400
+    times, when every partial took them)."""
+    from moba_hip.merge import merge_forward
+    g = torch.Generator().manual_seed(kmax)
+    T, H, D, M = 4096, 2, 64, 100_003
+    j = np.arange(M)
+    mapping = {"one": np.full(M, 777), "two in turn": j % 2 * 256, "sixteen in turn": j % 16 * 100,
+               "runs of ten": j // 10 % (T * H),
+               "one among many": np.where(j % 3 == 0, 4097, j % (T * H))}[rows]
+    so, ro = torch.randn(T, H, D, generator=g).cuda(), torch.randn(M, D, generator=g).cuda()
+    sl, rl = torch.randn(T, H, generator=g).cuda(), torch.randn(M, generator=g).cuda()
+
+    def call(m):
+        m = torch.from_numpy(m).int().cuda()
+        best = []
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            out = merge_forward(so, sl, ro, rl, m, kmax=kmax, check_capacity=False)
+            b.record()
+            torch.cuda.synchronize()
+            best.append(a.elapsed_time(b))
+        return out, min(best)
+    (out, lse), took = call(mapping)
+    order = np.argsort(mapping, kind="stable")
+    start = np.searchsorted(mapping[order], mapping[order], "left")
+    keep = np.sort(order[np.arange(M) - start < kmax])
+    ref = _ref(so, sl, ro[keep], rl[keep], torch.from_numpy(mapping[keep]))
+    np.testing.assert_allclose(out.double().cpu().numpy(), ref[0], atol=2e-6, rtol=1e-5)
+    np.testing.assert_allclose(lse.double().cpu().numpy(), ref[1], atol=2e-6, rtol=1e-6)
+    _, spread = call(np.random.default_rng(0).permutation(M) % (T * H))
+    assert took <= 10 * spread, f"{took * 1e3:.0f} us against {spread * 1e3:.0f}"
