@@ -143,26 +143,26 @@ class PrefillPlan:
         bit 1: remote), where 64-key tiles gain over 32-key ones.  ``longest``
         and ``keys``: keys of the longest self tile and of all of them.
 
+        From 384 keys on: with fewer the gain is about a microsecond (full
+        causal, 8 heads, D 128: 256 tokens 11.9 -> 10.8 us, 512 18.0 -> 15.9).
+
         Self: ``n`` counts the tiles of triangles of the longest one's height
         that hold as many keys.  Up to 128 dims a CU holds two 64-key
-        workgroups (three of 32 keys): up to 512 tiles they gain from 256 keys on
-        (16 tiles of up to 256 keys 11.9 -> 10.6 us; 512 of 128: 15.6 -> 16.5);
-        with more, the length from which they do doubles every 110 tiles: 768
-        tiles of up to 1024 keys 45.7 -> 48.9, of 2048 75.4 -> 72.8, of 4096 132
-        -> 118; 1024 tiles of up to 4096 166 -> 174, of 8192 301 -> 273.  Above
-        128 dims a CU holds one (two of 32 keys): 376 tiles of up to 6000 keys
-        271 -> 253, 384 of 2048 100.8 -> 99.9, 512 of 16384 761 -> 1017, of 2048
-        109 -> 141.
+        workgroups (three of 32 keys): up to 512 tiles they gain, with more the
+        length from which they do doubles every 110 tiles: 512 tiles of up to
+        128 keys 15.6 -> 16.5 us, 768 of up to 1024 45.7 -> 48.9, of 2048 75.4 ->
+        72.8, of 4096 132 -> 118; 1024 of up to 4096 166 -> 174, of 8192 301 ->
+        273.  Above 128 dims a CU holds one (two of 32 keys): 376 tiles of up to
+        6000 keys 271 -> 253, 384 of 2048 100.8 -> 99.9, 512 of 16384 761 -> 1017,
+        of 2048 109 -> 141.
 
         Remote, up to 128 dims: all tiles at once on two per CU (chunk 1024: 480
         tiles 74.1 -> 72.1, 672 91.7 -> 96.9; chunk 512: 480 47.8 -> 46.6, 585
-        55.1 -> 58.6), and chunks long enough to tell (256: 398 tiles 35.0 ->
-        33.5; 64: 94 tiles 16.4 -> 16.2)."""
+        55.1 -> 58.6)."""
         n = 2 * keys / longest
         wide = self.head_dim > 128
-        most = 448 if wide else 512 + 110 * math.log2(max(1, longest / 256))
-        self_bit = longest >= 256 and n <= most
-        remote_bit = self.remote > 0 and not wide and chunk >= 256 and self.max_remote_tiles <= 512
+        self_bit = longest >= 384 and n <= (448 if wide else 512 + 110 * math.log2(longest / 256))
+        remote_bit = self.remote > 0 and not wide and chunk >= 384 and self.max_remote_tiles <= 512
         return int(self_bit) | 2 * int(remote_bit)
 
     def _workspaces(self):

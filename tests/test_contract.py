@@ -240,9 +240,9 @@ def test_plan_cache_is_thread_safe():
     ((8192,), 16, 16, 128, 512, 1, 1), ((12000,) + (300,) * 100, 4, 4, 128, 512, 1, 1),
     ((6000,), 8, 8, 192, 512, 1, 1), ((2048,) * 3, 8, 8, 136, 512, 1, 1),
     ((2048,) * 4, 8, 8, 136, 512, 1, 0), ((16384,), 4, 4, 256, 512, 1, 0),
-    # remote tiles: 384, 672 and 398 of them, short chunks, wide heads
+    # remote tiles: 384, 672 and 288 of them, a short chunk, wide heads
     ((4096,), 8, 8, 128, 1024, 3, 3), ((4096,), 14, 14, 128, 1024, 3, 1),
-    ((2048,), 12, 2, 128, 256, 3, 3), ((1024,), 4, 2, 128, 64, 3, 0),
+    ((2048,), 12, 2, 128, 512, 3, 3), ((2048,), 12, 2, 128, 300, 3, 0),
     ((4096,), 2, 2, 192, 1024, 3, 1), ((4096,), 16, 4, 192, 1024, 3, 0),
 ])
 def test_long_tile_hint(lens, hq, hkv, dim, chunk, topk, hint):

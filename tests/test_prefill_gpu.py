@@ -619,7 +619,7 @@ def test_largest_weight_is_not_rounded(cuda_device, dtype, dim, remote):
 @pytest.mark.parametrize("dim", [72, 96, 120, 128, 136, 192, 256])
 @pytest.mark.parametrize("topk,lens,chunk", [
     (1, (515, 33, 300), 512),     # partial 32- and 64-key tiles, sequences below one tile
-    (3, (1033, 70, 290), 260),    # a chunk end inside a tile, a last chunk below a tile
+    (3, (1233, 70, 433), 390),    # a chunk end inside a tile, a last chunk below a tile
 ])
 def test_64_key_tiles(cuda_device, dtype, dim, topk, lens, chunk):
     """The kernels of long tiles over dtypes and head dims (columns past D in
