@@ -495,12 +495,13 @@ def test_remote_tiles_given_or_searched(cuda_device, monkeypatch, hq, hkv, dim, 
 
 @pytest.mark.parametrize("dim", [40, 64, 128, 136, 256])
 @pytest.mark.parametrize("topk", [3, 9])
-@pytest.mark.parametrize("scale", [1e-20, 3e18])
+@pytest.mark.parametrize("scale", [1e-20, 3e18, 1e19, 3e19])
 def test_gate_bits_at_the_ends_of_the_range(cuda_device, dim, topk, scale):
-    """Gate chains whose products and sums are subnormal in fp32, and ones that
-    overflow on the way: every score has the oracle's bits, for both widths of
-    the selection registers, with more candidates than one 16-wide pass and
-    tokens on both sides of a 256-token block."""
+    """Gate chains whose products and sums are subnormal in fp32, ones near the
+    largest float, and ones that overflow on the way, some (1e19) or all of
+    them: every score has the oracle's bits, for both widths of the selection
+    registers, with more candidates than one 16-wide pass and tokens on both
+    sides of a 256-token block."""
     q, k, v, cu, ml, _ = prefill_inputs(4, 2, dim, (300, 37), torch.bfloat16, seed=31)
     q, k = q.detach() * scale, k.detach() * scale
     plan, rt, gate = _gpu_route(q, k, cu, {"chunk_size": 11, "topk": topk}, 1)
@@ -512,8 +513,47 @@ def test_gate_bits_at_the_ends_of_the_range(cuda_device, dim, topk, scale):
     np.testing.assert_array_equal(g[~nan].view(np.uint32), gate_ref[~nan].view(np.uint32))
     tiny = np.abs(gate_ref[~nan & np.isfinite(gate_ref)])
     assert scale > 1 or ((tiny > 0) & (tiny < 2.0 ** -126)).any()
-    if not nan.any():
-        np.testing.assert_array_equal(rt.sel.cpu().numpy(), sel)
+    legal = _legal(plan)
+    scores = np.where(legal[:, None], gate_ref, 0.0)
+    if scale >= 1e19:
+        assert (scores == np.inf).any() and (scores == -np.inf).any()
+        assert np.isfinite(gate_ref[legal[:, None].repeat(4, 1)]).any() == (scale < 3e19)
+    assert not nan.any()
+    rows = (scores > -np.inf).all(0).T      # [T, Hq]: no score that is never chosen
+    assert rows.any()
+    np.testing.assert_array_equal(rt.sel.cpu().numpy()[rows], sel[rows])
+
+
+def _legal(plan):
+    """[F, T]: the filtered chunk lies in the token's sequence, before its chunk."""
+    own = np.searchsorted(plan.cu_chunk, np.arange(plan.cu[-1]), "right") - 1
+    batch, f = np.array(plan.chunk_batch), np.array(plan.filtered)
+    return (batch[f][:, None] == batch[own][None]) & (f[:, None] < own[None])
+
+
+@pytest.mark.parametrize("dim", [40, 64, 136, 256])
+@pytest.mark.parametrize("topk", [3, 9])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gate_of_infinities_and_nan(cuda_device, dtype, dim, topk):
+    """Infinite and NaN queries and keys reach the scores of their own token or
+    chunk and no other: NaN exactly where the oracle has it, the oracle's bits
+    elsewhere, and its choice for every token whose scores can all be chosen."""
+    q, k, v, cu, ml, _ = prefill_inputs(4, 2, dim, (300, 37), dtype, seed=59)
+    inf, nan = float("inf"), float("nan")
+    q[70, 1, 3], q[255, 0, dim - 1], q[256, 3, 0], q[320, 2, 5] = inf, nan, -inf, inf
+    k[20, 0, 7], k[150, 1, dim - 1], k[151, 1, 2], k[152, 1, 2] = inf, nan, inf, -inf
+    plan, rt, gate = _gpu_route(q, k, cu, {"chunk_size": 11, "topk": topk}, 1)
+    sel, means, gate_ref, _ = oracle_route(q, k, cu, 11, topk, 1)
+    for got, ref in ((rt.means.cpu().numpy(), means), (gate.cpu().numpy(), gate_ref)):
+        bad = np.isnan(ref)
+        assert bad.any() and not bad.all()
+        np.testing.assert_array_equal(np.isnan(got), bad)
+        np.testing.assert_array_equal(got[~bad].view(np.uint32), ref[~bad].view(np.uint32))
+    scores = np.where(_legal(plan)[:, None], gate_ref, 0.0)
+    assert (scores == inf).any() and (scores == -inf).any()
+    rows = (scores > -inf).all(0).T
+    assert rows.any()
+    np.testing.assert_array_equal(rt.sel.cpu().numpy()[rows], sel[rows])
 
 
 @pytest.mark.parametrize("topk,hint", [(1, 1), (3, 3)])
