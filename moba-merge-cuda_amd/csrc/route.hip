@@ -207,11 +207,11 @@ __global__ __launch_bounds__(256) void route_kernel(const uint16_t* __restrict__
         const int r = i * 8 + (lane >> 3);
         st8(st + r * 64 + (((lane & 7) ^ ((r >> 1) & 7)) * 8), x[sl * 8 + i]);
       }
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_sync();
 #pragma unroll
       for (int i = 0; i < 8; ++i)
         qv[sl * 8 + i] = ld8(st + lane * 64 + ((i ^ ((lane >> 1) & 7)) * 8));
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_sync();
     }
   }
   // chunk containing s (the last token's for the threads past T)
