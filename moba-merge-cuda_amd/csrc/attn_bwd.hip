@@ -117,8 +117,8 @@ __device__ __forceinline__ void finish_row(const BwdArgs& a, f32x16_t (&acc)[DP 
   }
 }
 
-// Per wave two blocks of 32 query rows; K/V tiles of 64 keys double-buffered
-// in LDS (row-major).  S^T = K Q^T and dP^T = V dO^T take K / V rows as the A
+// Head dims up to 128.  Per wave QB blocks of 32 query rows; K/V tiles of 64 keys
+// double-buffered in LDS (row-major).  S^T = K Q^T and dP^T = V dO^T take K / V rows as the A
 // operand; dQ^T = K^T dS^T reads K^T with the transposed LDS read.
 template <int DT, int DP, bool REMOTE, int QB>
 __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a) {
@@ -439,9 +439,15 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
 // Role S goes first (s_setprio): role G's MFMAs run under its element-wise
 // work.  K has 4 stages and V 3 (t - 1, t, and two blocks of loads in flight);
 // one barrier a step.  The sums are those of dq_kernel, in its order.
-// T 8192, 16/4 heads, chunk 1024, top-3, D 256: remote 570 -> 425-454 us, self
-// 188 -> 195-205 us, the training step 1780 -> 1681 us; matrix units busy 44%
-// and 28% of the CU cycles, LDS 25% and 16% with no bank conflicts.  2 to 5
+// T 8192, 16/4 heads, chunk 1024, top-3, D 256: remote 570 -> 425-454 us, the
+// training step 1780 -> 1681 us; matrix units busy 44% of the CU cycles, LDS 25%
+// with no bank conflicts.  The self launch (matrix units 28%, LDS 16%) gains
+// where a few long tiles decide and loses where many tiles fill the CUs.  Full
+// causal attention, delta and dQ, one-wave body -> this, us: D 256, 4096 tokens,
+// 8 heads 185 -> 168, 32768, 4 heads 3713 -> 3560, 8192, 16/4 heads 873 -> 877,
+// 8 x 1024 169.5 -> 172, 16 x 512 130 -> 134; D 160, 8 x 1024 142 -> 148, 16 x
+// 512 105 -> 112 (with 8-byte rows, as both were before: 194, 3774, 899, 183.5,
+// 146; 160, 123).  2 to 5
 // (role S) or 4 to 8 (role G) operand reads in flight and no priority measure
 // the same, role G first 8% slower; the element-wise work of block t - 1 between
 // role S's MFMAs of block t (two S^T and dP^T in registers, five K stages) is

@@ -1,4 +1,5 @@
-// Key-major dK / dV of the MoBA prefill backward, one wave per SIMD.
+// Key-major dK / dV of the MoBA prefill backward for head dims up to 64: every
+// wave runs all four products for its keys, two waves per SIMD.
 //
 // Replaces the dk/dv halves of the two flash-attention backwards in
 // OptMixedAttention.backward (src/moba_opt/mixed_attention.py:165-221) and the
@@ -28,9 +29,10 @@
 // laid side by side in the wave's own stream: the first 32 rows' exponentials
 // between the second 32 rows' S / dP products, the second's between the
 // first's dV / dK products, with LDS operands read two steps ahead and the
-// mask behind a uniform branch (a second, masked body took 251 registers).  T 16384, 14/2 heads, chunk 2048: 735 -> 655 us; the ragged
-// fp16 batch of 12238 tokens, 28/4 heads: 331 -> 285 us (one body alone 690 /
-// 302; three or four steps ahead the same; tiles of 32 rows 750 / 330).
+// mask behind a uniform branch (a second, masked body took 251 registers).
+// T 16384, 14/2 heads, chunk 2048: 735 -> 655 us; the ragged fp16 batch of 12238
+// tokens, 28/4 heads: 331 -> 285 us (one body alone 690 / 302; three or four
+// steps ahead the same; tiles of 32 rows 750 / 330).
 #include <type_traits>
 
 #include "common.h"

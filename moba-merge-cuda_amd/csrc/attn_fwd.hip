@@ -66,8 +66,8 @@ struct FwdArgs {
 // Keys per LDS tile, and the waves per SIMD the registers are held to.  What
 // hides the latencies of a tile (LDS operands, exponentials, the barrier) is
 // another workgroup on the CU, so the tile is cut until one more fits: 32 keys
-// give three waves per SIMD at 128 dims (139 registers; 64 keys: two) and two
-// at 256 (242 registers, 64 KB of LDS; 64 keys: one wave, 128 KB).  Remote /
+// give three waves per SIMD at 128 dims (152 registers; 64 keys: two) and two
+// at 256 (256 registers, 64 KB of LDS; 64 keys: one wave, 128 KB).  Remote /
 // self forward, us, 64 -> 32 keys: T 32768, 32 heads, D 128, chunk 4096
 // 3570 / 1425 -> 3415 / 1346; T 8192, 16/4 heads, D 256, chunk 1024 455 / 206
 // -> 289 / 171.  A fourth wave at 128 dims spills and is slower (3510 / 1460),

@@ -1,5 +1,5 @@
 // Argument block of the prefill backward kernels (attn_bwd.hip, attn_dkdv.hip,
-// attn_dkdv2.hip).
+// attn_dkdv2.hip, attn_dkdv4.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -35,7 +35,7 @@ struct BwdArgs {
   float* lse_k;      // [T*Hq] lse / scale: the row's log-sum-exp in q.k units
   uint16_t* part_dq;  // remote dQ slots, input dtype
   // Row-split schedule (kv_splits > 1, built on the device by
-  // dkdv_sched_kernel): kv_sched[4 * workgroup] = (kv tile, first row tile,
+  // delta_sched_kernel or dkdv_sched_kernel): kv_sched[4 * workgroup] = (kv tile, first row tile,
   // end row tile, partial slot or -1 to write dK / dV directly), tile -1 for
   // an idle workgroup; kv_seg[2 * kv tile] = (first slot, slots).  part_dkv
   // holds per slot [dK | dV][128 keys][D] fp32, summed by dkdv_reduce_kernel.

@@ -257,19 +257,10 @@ MOBA_DEV void dma_lds4(__amdgpu_buffer_rsrc_t r, const void* lds, uint32_t voff,
                :: "s"(lds_addr(lds)), "v"(voff), "s"(r), "s"(soff) : "memory", "m0");
 }
 
-// Workgroup barriers for kernels whose LDS tiles arrive by buffer loads.
-// The empty asm statements keep the compiler from moving memory accesses
-// across the barrier; the explicit waits are visible to its wait-count pass.
-//   stage_barrier: this wave's buffer loads (and LDS accesses) complete, then
-//                  the barrier: every wave's loads have landed after it.
-//   lds_barrier:   LDS accesses complete, then the barrier; buffer loads in
-//                  flight stay in flight.
-MOBA_DEV void stage_barrier() {
-  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
+// Workgroup barrier for kernels whose LDS tiles arrive by buffer loads: LDS
+// accesses complete, buffer loads in flight stay in flight.  The empty asm
+// statements keep the compiler from moving memory accesses across the barrier;
+// the explicit wait is visible to its wait-count pass.
 MOBA_DEV void lds_barrier() {
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
   asm volatile("" ::: "memory");
@@ -394,18 +385,6 @@ MOBA_DEV float canon_tree(float v) {
   for (int off = 32; off > 0; off >>= 1) v = v + __shfl_down(v, off, 64);
   return v;
 }
-
-MOBA_DEV float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
-MOBA_DEV float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
 
 // acc[k] = fma(lane (row base + J0 + j) of b[k], m[j], acc[k]) for j = 0..7 in
 // order, four independent chains k interleaved (so consecutive instructions
