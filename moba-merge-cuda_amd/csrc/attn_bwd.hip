@@ -440,8 +440,8 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
 // work.  K has 4 stages and V 3 (t - 1, t, and two blocks of loads in flight);
 // one barrier a step.  The sums are those of dq_kernel, in its order.
 // T 8192, 16/4 heads, chunk 1024, top-3, D 256: remote 570 -> 425-454 us, the
-// training step 1780 -> 1681 us; matrix units busy 44% of the CU cycles, LDS 25%
-// with no bank conflicts.  The self launch (matrix units 28%, LDS 16%) gains
+// training step 1780 -> 1681 us; matrix units busy 39% of the cycles, LDS 22%
+// with no bank conflicts.  The self launch (matrix units 24%, LDS 14%) gains
 // where a few long tiles decide and loses where many tiles fill the CUs.  Full
 // causal attention, delta and dQ, one-wave body -> this, us: D 256, 4096 tokens,
 // 8 heads 185 -> 168, 32768, 4 heads 3713 -> 3560, 8192, 16/4 heads 873 -> 877,
