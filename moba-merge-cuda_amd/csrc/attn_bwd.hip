@@ -8,7 +8,7 @@
 // GQA gradients of the heads sharing a KV head are summed.
 //
 //   delta_kernel : Delta = rowsum(dO * O)                                  [T*Hq]
-//   dq_kernel<REMOTE> (dq2_kernel above 128 dims) : query-major.  S^T = K Q^T, dP^T = V dO^T,
+//   dq_kernel<REMOTE> (dq2_kernel above 128 dims, self above 192) : query-major.  S^T = K Q^T, dP^T = V dO^T,
 //        P = exp(S*scale - LSE), dS = P (dP - Delta), dQ^T += K^T dS^T.
 //        REMOTE tiles (expert rows) write dq partials into the row's slot;
 //        SELF tiles (causal within the chunk) add the slots in ascending order.
@@ -117,13 +117,15 @@ __device__ __forceinline__ void finish_row(const BwdArgs& a, f32x16_t (&acc)[DP 
   }
 }
 
-// Head dims up to 128.  Per wave QB blocks of 32 query rows; K/V tiles of 64 keys
-// double-buffered in LDS (row-major).  S^T = K Q^T and dP^T = V dO^T take K / V rows as the A
+// Head dims up to 128, and the self launch up to 192 (dq2_kernel has the others).
+// Per wave QB blocks of 32 query rows; K/V tiles of 64 keys double-buffered in
+// LDS (row-major).  S^T = K Q^T and dP^T = V dO^T take K / V rows as the A
 // operand; dQ^T = K^T dS^T reads K^T with the transposed LDS read.
 template <int DT, int DP, bool REMOTE, int QB>
 __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a) {
   constexpr int NKS = DP / 16, NDB = DP / 32;
   constexpr int TILE = kBN * DP, NB = DP / 8, NDMA = kBN * NB / 256;
+  static_assert(DP <= 128 || !REMOTE, "dq2_kernel has the remote launch of the wide heads");
   // Two stages of K and V tiles (swz<DP> layout) filled by buffer loads
   // straight into LDS, as in the forward kernel.
   __shared__ __attribute__((aligned(16))) uint16_t K0[TILE];
@@ -181,13 +183,19 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
   const int wave_s = __builtin_amdgcn_readfirstlane(wave);
   // Lane l of wave w loads blocks j = (n * 4 + w) * 64 + l: row j / NB,
   // physical block j % NB.  The row advances by 256 / NB per n, a multiple of
-  // 16, and the swizzle depends on the row mod 16 only, so every n has the
-  // same column and its offset is the n = 0 offset plus a uniform step (added
-  // per load, not held in NDMA registers).
-  static_assert((256 / NB) % 16 == 0, "head dims up to 128");
-  const int vj = wave_s * 64 + lane, vrow = vj / NB;
-  const int vcol = swz<DP>(vrow, (vj % NB) * 8) - vrow * DP;  // swizzle is an involution
-  const uint32_t voff = (uint32_t)(((vrow * a.Hkv + kh) * D + vcol) * 2);
+  // 16 up to 128 dims, and the swizzle depends on the row mod 16 only, so every n
+  // has the same column and its offset is the n = 0 offset plus a uniform step
+  // (added per load, not held in NDMA registers).
+  constexpr bool UNI = (256 / NB) % 16 == 0;
+  uint32_t voff[UNI ? 1 : NDMA];
+  bool vok[UNI ? 1 : NDMA];
+#pragma unroll
+  for (int n = 0; n < (UNI ? 1 : NDMA); ++n) {
+    const int j = (n * 4 + wave_s) * 64 + lane, row = j / NB;
+    const int col = swz<DP>(row, (j % NB) * 8) - row * DP;  // swizzle is an involution
+    voff[n] = (uint32_t)(((row * a.Hkv + kh) * D + col) * 2);
+    vok[n] = col < D;
+  }
   const uint32_t vstep = (uint32_t)((256 / NB) * a.Hkv * D * 2);
   const int n_keys = k_hi - k_lo;
   const uint32_t nrec = (uint32_t)((((int64_t)(n_keys - 1) * a.Hkv + kh + 1) * D) * 2);
@@ -196,11 +204,11 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
   const uint32_t tile_bytes = (uint32_t)(kBN * a.Hkv * D * 2);
   auto dma = [&](uint16_t* Kd, uint16_t* Vd, int it) {
     const uint32_t soff = (uint32_t)it * tile_bytes;
-    const uint32_t v0 = opaque(voff);
+    const uint32_t v0 = opaque(voff[0]);
 #pragma unroll
     for (int n = 0; n < NDMA; ++n) {
-      if (vcol < D) {
-        const uint32_t vo = v0 + n * vstep;
+      if (vok[UNI ? 0 : n]) {
+        const uint32_t vo = UNI ? v0 + n * vstep : voff[n];
         load_lds16(make_rsrc(kbase, nrec), Kd + (n * 4 + wave_s) * 64 * 8, vo, soff);
         load_lds16(make_rsrc(vbase, nrec), Vd + (n * 4 + wave_s) * 64 * 8, vo, soff);
       }
@@ -216,9 +224,12 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
     __syncthreads();
   }
   // The first K / V tile goes out before the query rows: an expert's rows
-  // wait for their row list, the tile only for the workgroup's entry.  Rows
-  // past the tile's end load the last row's data and are never written.
-  dma(K0, V0, 0);
+  // wait for their row list, the tile only for the workgroup's entry (above 128
+  // dims the rows come first and each load is guarded: otherwise the kernel
+  // spills 325 registers).  Rows past the tile's end load the last row's data
+  // and are never written.
+  constexpr bool TILE_FIRST = DP <= 128;
+  if constexpr (TILE_FIRST) dma(K0, V0, 0);
   u16x8_t qf[QB][NKS], gf[QB][NKS];
   float lse2[QB], lk[QB], dl[QB];
 #pragma unroll
@@ -233,9 +244,14 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
       const int d = ks * 16 + hh * 8, dc = d < D ? d : 0;
-      const u16x8_t xq = ld8(a.q + row * D + dc), xg = ld8(a.dout + row * D + dc);
-      qf[qb][ks] = d < D ? xq : zero8();
-      gf[qb][ks] = d < D ? xg : zero8();
+      if constexpr (TILE_FIRST) {
+        const u16x8_t xq = ld8(a.q + row * D + dc), xg = ld8(a.dout + row * D + dc);
+        qf[qb][ks] = d < D ? xq : zero8();
+        gf[qb][ks] = d < D ? xg : zero8();
+      } else {
+        qf[qb][ks] = valid[qb] && d < D ? ld8(a.q + row * D + d) : zero8();
+        gf[qb][ks] = valid[qb] && d < D ? ld8(a.dout + row * D + d) : zero8();
+      }
     }
     const float lr = a.lse[row];
     lse2[qb] = lr * kLog2e;
@@ -266,6 +282,7 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
     }
   }
 
+  if constexpr (!TILE_FIRST) dma(K0, V0, 0);
   const uint32_t kbase0 = swz_b128_base<DP>(lane);
   const uint32_t trb0 = swz_tr_base<DP>(lane, 0), trb1 = swz_tr_base<DP>(lane, 1);
 
@@ -441,13 +458,11 @@ __global__ __launch_bounds__(256, attn_occupancy<DP>()) void dq_kernel(BwdArgs a
 // one barrier a step.  The sums are those of dq_kernel, in its order.
 // T 8192, 16/4 heads, chunk 1024, top-3, D 256: remote 570 -> 425-454 us, the
 // training step 1780 -> 1681 us; matrix units busy 39% of the cycles, LDS 22%
-// with no bank conflicts.  The self launch (matrix units 24%, LDS 14%) gains
-// where a few long tiles decide and loses where many tiles fill the CUs.  Full
-// causal attention, delta and dQ, one-wave body -> this, us: D 256, 4096 tokens,
-// 8 heads 185 -> 168, 32768, 4 heads 3713 -> 3560, 8192, 16/4 heads 873 -> 877,
-// 8 x 1024 169.5 -> 172, 16 x 512 130 -> 134; D 160, 8 x 1024 142 -> 148, 16 x
-// 512 105 -> 112 (with 8-byte rows, as both were before: 194, 3774, 899, 183.5,
-// 146; 160, 123).  2 to 5
+// with no bank conflicts.  The self launch (above 192 dims; matrix units
+// 24%, LDS 14%) gains over one wave per 32 rows where a few long tiles decide and
+// loses where many tiles fill the CUs: full causal attention, D 256, delta and
+// dQ, us: 4096 tokens, 8 heads 185 -> 168, 32768, 4 heads 3713 -> 3560, 8192,
+// 16/4 heads 873 -> 877, 8 x 1024 169.5 -> 172, 16 x 512 130 -> 134.  2 to 5
 // (role S) or 4 to 8 (role G) operand reads in flight and no priority measure
 // the same, role G first 8% slower; the element-wise work of block t - 1 between
 // role S's MFMAs of block t (two S^T and dP^T in registers, five K stages) is
@@ -625,11 +640,20 @@ __global__ __launch_bounds__(512, 2) void dq2_kernel(BwdArgs a) {
   }
 }
 
+// Up to 192 dims the causal launch is faster with one wave per 32 rows (64-key
+// tiles, half the barriers): delta and dQ, full causal, 16/4 heads, dq2_kernel ->
+// this, us: 16 x 512 tokens D 136 107 -> 98, D 160 111 -> 104, D 192 118.5 ->
+// 113.5; 2 x 4096 D 192 392 -> 383; 4096 tokens, 8 heads, D 192 166 -> 167.  At
+// 224 both are within 2.5% either way, at 256 see dq2_kernel.
 template <int DT, int DP, bool REMOTE>
 void launch_dq(const BwdArgs& a, unsigned grid, hipStream_t st) {
-  if constexpr (DP <= 128)
-    hipLaunchKernelGGL((dq_kernel<DT, DP, REMOTE, attn_qb<DP>()>), dim3(grid), dim3(256), 0, st, a);
-  else
+  if constexpr (DP <= 128 || !REMOTE) {
+    if (DP <= 128 || a.D <= 192) {
+      hipLaunchKernelGGL((dq_kernel<DT, DP, REMOTE, attn_qb<DP>()>), dim3(grid), dim3(256), 0, st, a);
+      return;
+    }
+  }
+  if constexpr (DP > 128)
     hipLaunchKernelGGL((dq2_kernel<DT, DP, REMOTE>), dim3(grid), dim3(512), 0, st, a);
 }
 
