@@ -54,14 +54,15 @@ __global__ __launch_bounds__(256) void merge_init_kernel(int* slots, int64_t P, 
 // So a wave's lanes of one row are found (each leaves its number at a hash of
 // its row; a lane that reads another lane of its row there has company) and
 // numbered: the lane of rank r has r smaller indices beside it, so it can start
-// at slot r, and from rank kmax on it is not among the row's first kmax.  Such
-// lanes look before each minimum, and every lane that two slots have turned away
-// looks at the last: a slot only ever falls, so one that reads below x, be it
-// stale, will not take x.
+// at slot r, and from rank kmax on it is not among the row's first kmax.  From
+// four of them on they look before each minimum (fewer meet by chance, and a
+// look is a memory latency): a slot only ever falls, so one that reads below x,
+// be it stale, will not take x.
 // Whole call, 344K partials, kmax 8, us, without -> with this (the radix sort
-// took 590 in each case): one row 31256 -> 111, every other partial of one row
-// 15657 -> 158, 64 rows in turn (never two in a wave) 663 -> 743, spread 73 ->
-// 73; T 16384, 14 heads, kmax 2: 69.1 -> 69.5.
+// took 590 in each case): one row 31247 -> 179, every other partial of one row
+// 15654 -> 256, 16 rows in turn 2014 -> 342, 64 rows in turn (never two in a
+// wave) 665 -> 665, sorted runs of eight 139 -> 67, spread 79 -> 79; T 16384, 14
+// heads, kmax 2: 67.3 -> 67.4.
 constexpr int kRowHash = 256;
 
 template <typename MT>
@@ -80,29 +81,40 @@ __global__ __launch_bounds__(256) void merge_insert_kernel(const MT* __restrict_
   wave_lds_sync();
   const int mate = ok ? *at : lane;
   const bool met = __shfl(p, mate, 64) == p && mate != lane;  // -1: its own lane
-  int rank = 0;
-  bool crowd = false;
-  for (uint64_t todo = __ballot(met); todo != 0;) {
-    const bool mine = p == __builtin_amdgcn_readlane(p, __ffsll((unsigned long long)todo) - 1);
-    const uint64_t row = __ballot(mine);
-    if (mine) {
-      rank = __popcll(row & ((1ull << lane) - 1ull));
-      crowd = true;
+  int* row = slots + (int64_t)p * kmax;
+  int x = (int)j, i = 0;
+  uint64_t todo = __ballot(met);
+  if (todo != 0) {  // uniform
+    bool crowd = false;
+    for (; todo != 0;) {
+      const bool mine = p == __builtin_amdgcn_readlane(p, __ffsll((unsigned long long)todo) - 1);
+      const uint64_t mates = __ballot(mine);
+      if (mine) {
+        i = __popcll(mates & ((1ull << lane) - 1ull));
+        crowd = __popcll(mates) >= 4;
+      }
+      todo &= ~mates;
     }
-    todo &= ~row;
+    auto look = [&](int k) { return __hip_atomic_load(row + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    if (crowd) {
+      if (i < kmax && look(kmax - 1) < x) i = kmax;
+      for (; i < kmax; ++i) {
+        if (look(i) < x) continue;
+        const int old = atomicMin(row + i, x);
+        x = max(old, x);
+        if (x == kEmpty) return;
+      }
+      status[1] = 1;  // more than kmax: an index has no slot
+      return;
+    }
   }
   if (!ok) return;
-  int* row = slots + (int64_t)p * kmax;
-  auto look = [&](int i) { return __hip_atomic_load(row + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-  int x = (int)j;
-  for (int i = rank; i < kmax; ++i) {
-    if (i == (crowd ? rank : 2) && look(kmax - 1) < x) break;
-    if (crowd && look(i) < x) continue;
+  for (; i < kmax; ++i) {
     const int old = atomicMin(row + i, x);
     x = max(old, x);
     if (x == kEmpty) return;
   }
-  status[1] = 1;  // more than kmax: an index has no slot
+  status[1] = 1;
 }
 
 // 16 bytes of a row: 8 elements (16-bit types) or 4 (fp32).
